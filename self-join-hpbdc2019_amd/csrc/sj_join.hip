@@ -2592,64 +2592,6 @@ sj_status join(sj_grid_s *g, const sj_join_params *P, sj_result_s *r) {
     return SJ_OK;
 }
 
-// ------------------------------------------------------- canonical rows
-// Rows sorted ascending, one wave per row: rows up to 1024 entries by a
-// bitonic sort in LDS, longer rows by a serial shell sort (rare).
-constexpr int SR_CAP = 1024;
-
-__global__ __launch_bounds__(256) void k_sort_rows(const uint64_t *offsets, int32_t *ids, uint64_t n,
-                                                   uint64_t base, uint64_t idsCap) {
-    __shared__ int32_t buf[4][SR_CAP];
-    const unsigned wave = threadIdx.x >> 6, lane = __lane_id();
-    const uint64_t row = (uint64_t)blockIdx.x * 4 + wave;
-    if (row >= n) return;
-    if (idsCap && offsets[n] - base > idsCap) return;  // the fill wrote nothing
-    const uint64_t b = offsets[row] - base, e = offsets[row + 1] - base;
-    const uint64_t len = e - b;
-    if (len < 2) return;
-    if (len <= SR_CAP) {
-        uint32_t p2 = 2;
-        while (p2 < len) p2 <<= 1;
-        for (uint32_t i = lane; i < p2; i += 64) buf[wave][i] = i < len ? ids[b + i] : INT32_MAX;
-        wave_lds_sync();
-        for (uint32_t kk = 2; kk <= p2; kk <<= 1) {
-            for (uint32_t jj = kk >> 1; jj > 0; jj >>= 1) {
-                for (uint32_t i = lane; i < p2; i += 64) {
-                    const uint32_t l = i ^ jj;
-                    if (l > i) {
-                        const int32_t x = buf[wave][i], y = buf[wave][l];
-                        const bool up = (i & kk) == 0;
-                        if ((x > y) == up) {
-                            buf[wave][i] = y;
-                            buf[wave][l] = x;
-                        }
-                    }
-                }
-                wave_lds_sync();
-            }
-        }
-        for (uint32_t i = lane; i < len; i += 64) ids[b + i] = buf[wave][i];
-    } else if (lane == 0) {
-        int32_t *v = ids + b;
-        for (uint64_t gap = len / 2; gap > 0; gap /= 2)
-            for (uint64_t i = gap; i < len; i++) {
-                int32_t x = v[i];
-                uint64_t j = i;
-                for (; j >= gap && v[j - gap] > x; j -= gap) v[j] = v[j - gap];
-                v[j] = x;
-            }
-    }
-}
-
-sj_status sort_rows_device(sj_context ctx, const uint64_t *offsets, int32_t *ids, uint64_t n, uint64_t base,
-                           uint64_t idsCap) {
-    if (!n) return SJ_OK;
-    hipLaunchKernelGGL(k_sort_rows, dim3((unsigned)((n + 3) / 4)), dim3(256), 0, ctx->stream, offsets, ids, n,
-                       base, idsCap);
-    SJ_LAUNCH_CHECK();
-    return SJ_OK;
-}
-
 // Original-ID-order CSR from the cell-order table (on demand).
 __global__ void k_row_lengths_orig(const uint64_t *off, const uint32_t *rowIds, uint64_t n, uint32_t *len) {
     uint64_t r = (uint64_t)blockIdx.x * JB + threadIdx.x;

@@ -101,7 +101,9 @@ typedef struct sj_stats {
     uint64_t num_batches;
     uint64_t candidates;         /* distance evaluations of the count pass */
     uint64_t fp32_band_pairs;    /* candidates re-decided in FP64 */
-    uint64_t fp32_misclassified; /* pairs whose plain FP32 decision was wrong */
+    uint64_t fp32_misclassified; /* pairs whose plain FP32 decision was wrong
+                                  * (d = k >= 4: those the FP32 filter passed
+                                  * and FP64 rejected) */
     uint64_t overflow_retries;
     double ms_grid;              /* device time, grid construction */
     double ms_workload;          /* device time, workload estimate + order */

@@ -223,6 +223,7 @@ struct sj_grid_s {
     sj::DBuf<uint32_t> cellCoord;    // nNonEmpty x k
     sj::DBuf<uint32_t> posLB;        // totalCells+1 (dense grids): first sorted position with linear ID >= L
     sj::DBuf<float> sortedPts32;     // lazily built for the FP32 form
+    sj::DBuf<uint32_t> posPk;        // span walk (d = k >= 4): cell coordinates modulo 4 per sorted position
     double ms_build = 0.0;
     bool transient = false;          // made for one join, which may take its buffers
     // arena mode: device bytes the join still needs after the grid; the

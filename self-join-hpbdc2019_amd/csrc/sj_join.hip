@@ -28,9 +28,11 @@
 #include <cmath>
 #include <cstring>
 #include <memory>
+#include <type_traits>
 
 #include "sj_common.hpp"
 #include "sj_mfma.hpp"
+#include "sj_span.hpp"
 #include "sj_traverse.hpp"
 #include "sj_wide.hpp"
 
@@ -206,7 +208,7 @@ __device__ __forceinline__ void process_point(const JoinArgs &a, uint32_t s, Lan
 template <int D, int PREC>
 struct TileCfg {
     static constexpr int DD = D > 0 ? D : 1;
-    static constexpr int CH = D <= 4 ? 256 : 128;  // staged candidates per chunk
+    static constexpr int CH = 256;  // staged candidates per chunk
     static constexpr int MW = CH / 64;                              // mask words per lane (<= 4)
 };
 
@@ -226,18 +228,6 @@ struct TileLds {
 // most OWN_STAGE), then stored 64 consecutive entries at a time.
 constexpr uint32_t OWN_STAGE = 384;
 
-// LDS of a count pass: the staged coordinates and the mirrored-hit
-// counters (the candidate IDs and reservation slots belong to the fills).
-template <int D, int PREC>
-struct TileLdsCount {
-    using C = TileCfg<D, PREC>;
-    double x64[PREC == 1 ? 1 : C::CH + 64][C::DD];
-    float x32[PREC == 1 ? C::CH + 64 : 1][C::DD];
-    int32_t id[1];
-    uint32_t cnt[C::CH];
-    unsigned long long base[1];
-};
-
 // LDS of the fill that replays a hit record: candidate IDs and mirrored-hit
 // counters, chunked like the count pass of precision PREC, and the own-hit
 // stage: entry i is neighbour ID sid[i] for position wc[l] + t of lane l's
@@ -252,52 +242,6 @@ struct TileLdsIds {
     int32_t sid[OWN_STAGE];
     uint32_t sdst[OWN_STAGE];
 };
-
-// Upper bound of the pieces a tile walk executes: per neighbour row in the
-// grid, ceil(staged candidates / cw).  LDS tile walk: cw = 64 (chunks are
-// whole multiples of 64 candidates, a chunk runs at most ceil(chunk / 64)
-// pieces); matrix-core walk: cw = 32, one piece per 32-candidate chunk.
-template <int K>
-__device__ __forceinline__ uint32_t tile_piece_bound(const JoinArgs &a, const uint32_t *c, uint64_t rowBase,
-                                                     uint32_t xa, uint32_t xb, uint32_t cw) {
-    const uint32_t nC0 = a.nCells[0];
-    const uint32_t ux0 = xa >= 1 ? xa - 1 : 0u;
-    const uint32_t ux1 = xb + 1 < nC0 ? xb + 1 : nC0 - 1;
-    int o[K];
-#pragma unroll
-    for (int j = 0; j < K; j++) o[j] = -1;
-    int nrow = 1;
-#pragma unroll
-    for (int j = 1; j < K; j++) nrow *= 3;
-    uint32_t bound = 0;
-    for (int it = 0; it < nrow; ++it) {
-        bool inb = true;
-        int64_t dl = 0;
-#pragma unroll
-        for (int j = 1; j < K; j++) {
-            const int64_t v = (int64_t)c[j] + o[j];
-            inb = inb && v >= 0 && v < (int64_t)a.nCells[j];
-            dl += (int64_t)o[j] * a.mult[j];
-        }
-        if (inb) {
-            const uint64_t rb = (uint64_t)((int64_t)rowBase + dl);
-            bound += (pos_lb(a, rb + ux1 + 1) - pos_lb(a, rb + ux0) + cw - 1u) / cw;
-        }
-        bool carry = true;
-#pragma unroll
-        for (int j = 1; j < K; j++) {
-            if (carry) {
-                if (o[j] == 1) {
-                    o[j] = -1;
-                } else {
-                    o[j]++;
-                    carry = false;
-                }
-            }
-        }
-    }
-    return bound;
-}
 
 // One tile of <= 64 points of one cell row against its 3^(k-1) neighbour
 // rows.  RP (fill only): take the hit masks from the count pass's record
@@ -429,22 +373,12 @@ __device__ __forceinline__ void process_tile(const JoinArgs &a, uint32_t tile, L
     };
 
     // One neighbour row at offsets o[1..K-1] (o[0] unused) with cell-row
-    // base rb; the caller may pass the union's bounds [pu0, pu1) (given).
-    // Every lane shares the row coordinates, so control flow is uniform.
-    auto row = [&](const int (&o)[K], uint64_t rb, bool originRow, bool given, uint32_t pu0,
-                   uint32_t pu1) __attribute__((always_inline)) {
+    // base rb.  Every lane shares the row coordinates, so control flow is
+    // uniform.
+    auto row = [&](const int (&o)[K], uint64_t rb, bool originRow) __attribute__((always_inline)) {
         // claimed dim-0 offsets of this lane's cell in this row
         bool useL = false, useC = false, useR = false;
-        // every lane claims every cell of the row: a lane's span has no
-        // unclaimed gap (uniform)
-        const bool allClaimed = given && !originRow && a.form != SJ_FORM_BUNICOMP;
-        if (valid && allClaimed) {
-            // a row the lookup kept off the origin row: under FULL, LID and
-            // Unicomp every lane claims every cell of it
-            useL = x >= 1;
-            useC = true;
-            useR = x + 1 < nC0;
-        } else if (valid) {
+        if (valid) {
             int oo[K];
 #pragma unroll
             for (int j = 0; j < K; j++) oo[j] = o[j];
@@ -456,30 +390,10 @@ __device__ __forceinline__ void process_tile(const JoinArgs &a, uint32_t tile, L
             useC = originRow || claims<K>(a.form, c, oo, linA, rb + x);
         }
         if (__ballot(useL || useC || useR)) {
-            const uint32_t u0 = given ? pu0 : pos_lb_t<DN>(a, rb + ux0);
-            const uint32_t u1 = given ? pu1 : pos_lb_t<DN>(a, rb + ux1 + 1);
+            const uint32_t u0 = pos_lb_t<DN>(a, rb + ux0);
+            const uint32_t u1 = pos_lb_t<DN>(a, rb + ux1 + 1);
             uint32_t e0 = 0, e1 = 0, e2 = 0, e3 = 0;
-            // given: the first chunk is staged while the window bounds load
-            // (both requests in flight together); the lookups run on every
-            // lane, clamped to the row, and past-the-end lanes drop them
-            bool staged0 = false;
-            if (given) {
-                const uint32_t xl = x >= 1 ? x - 1 : x;
-                const uint32_t xr = x + 1 < nC0 ? x + 2 : x + 1;
-                const uint32_t f0 = pos_lb_t<DN>(a, rb + xl), f1 = pos_lb_t<DN>(a, rb + x);
-                const uint32_t f2 = pos_lb_t<DN>(a, rb + x + 1), f3 = pos_lb_t<DN>(a, rb + xr);
-                if constexpr (!RP) {
-                    const uint32_t m0 = min((uint32_t)CH, u1 - u0);
-                    if (!(PASS == PASS_FILL && !anyOwnW && (u0 + m0 <= a.wBegin || u0 >= a.wEnd))) {
-                        stage(u0, m0);
-                        staged0 = true;
-                    }
-                }
-                e0 = valid ? f0 : 0u;
-                e1 = valid ? f1 : 0u;
-                e2 = valid ? f2 : 0u;
-                e3 = valid ? f3 : 0u;
-            } else if (valid) {
+            if (valid) {
                 e1 = pos_lb_t<DN>(a, rb + x);
                 e2 = pos_lb_t<DN>(a, rb + x + 1);
                 e0 = x >= 1 ? pos_lb_t<DN>(a, rb + x - 1) : e1;
@@ -499,7 +413,7 @@ __device__ __forceinline__ void process_tile(const JoinArgs &a, uint32_t tile, L
                 const uint32_t chi = min(hi, c0 + m);
                 const uint32_t len = chi > clo ? chi - clo : 0u;
                 static_assert(CH <= 256, "lane spans need at most 9 bits");
-                const uint32_t maxLen = wave_max_small<CH == 256 ? 9 : 8>(len);
+                const uint32_t maxLen = wave_max_small<9>(len);
                 // replay: the chunk's recorded masks, requested before the
                 // staging so that both loads are in flight together
                 uint64_t rm[Cfg::MW];
@@ -554,7 +468,7 @@ __device__ __forceinline__ void process_tile(const JoinArgs &a, uint32_t tile, L
                         }
                     }
                 }
-                if (!(staged0 && c0 == u0)) stage(c0, m);
+                stage(c0, m);
                 wave_lds_sync();
                 // mirrored hits of the chunk, one word per 64-candidate piece
                 uint64_t mk0 = 0ull, mk1 = 0ull, mk2 = 0ull, mk3 = 0ull;
@@ -574,19 +488,15 @@ __device__ __forceinline__ void process_tile(const JoinArgs &a, uint32_t tile, L
                     uint64_t okm = 0ull;
                     uint32_t r0 = 0u;
                     if (base < len) {
-                        if (allClaimed) {
-                            okm = range_bits(pstart, pstart, clo + len);
-                        } else {
-                            if (useL) okm |= range_bits(pstart, e0, e1);
-                            if (useC) okm |= range_bits(pstart, e1, e2);
-                            if (useR) okm |= range_bits(pstart, e2, e3);
-                            okm &= range_bits(pstart, pstart, clo + len);
-                        }
+                        if (useL) okm |= range_bits(pstart, e0, e1);
+                        if (useC) okm |= range_bits(pstart, e1, e2);
+                        if (useR) okm |= range_bits(pstart, e2, e3);
+                        okm &= range_bits(pstart, pstart, clo + len);
                         r0 = pstart - c0;
                     }
                     // uniform trip count, US candidates per step, one bit
                     // per candidate; masks are applied per piece
-                    constexpr int US = D <= 3 ? 8 : 4;
+                    constexpr int US = 8;
                     for (uint32_t i = 0; i < n; i += US) {
                         uint32_t hb = 0u, mb = 0u;
 #pragma unroll
@@ -640,13 +550,8 @@ __device__ __forceinline__ void process_tile(const JoinArgs &a, uint32_t tile, L
                     // the rows written) and own hits of the piece
                     uint64_t mirBits = 0ull;
                     if (anyMirror) {
-                        // every hit is eligible when the lane claimed all cells
-                        // off the origin row
-                        uint64_t elig = ~0ull;
-                        if (!allClaimed) {
-                            elig = range_bits(pstart, e0, e1) | range_bits(pstart, e2, e3);
-                            if (mirC) elig |= range_bits(pstart, e1, e2);
-                        }
+                        uint64_t elig = range_bits(pstart, e0, e1) | range_bits(pstart, e2, e3);
+                        if (mirC) elig |= range_bits(pstart, e1, e2);
                         mirBits = mask & elig & range_bits(pstart, a.wBegin, a.wEnd);
                     }
                     const uint32_t myCnt = (uint32_t)__popcll(mask);
@@ -865,94 +770,32 @@ __device__ __forceinline__ void process_tile(const JoinArgs &a, uint32_t tile, L
         }
     };
 
-    if constexpr (K < 4) {
-        // neighbour rows one after another: odometer over dims 1..K-1
-        int o[K];
+    // neighbour rows one after another: odometer over dims 1..K-1
+    int o[K];
 #pragma unroll
-        for (int j = 0; j < K; j++) o[j] = -1;
-        o[0] = 0;
-        for (int it = 0; it < nrow; ++it) {
-            bool inb = true, originRow = true;
-            int64_t dl = 0;
+    for (int j = 0; j < K; j++) o[j] = -1;
+    o[0] = 0;
+    for (int it = 0; it < nrow; ++it) {
+        bool inb = true, originRow = true;
+        int64_t dl = 0;
 #pragma unroll
-            for (int j = 1; j < K; j++) {
-                originRow = originRow && o[j] == 0;
-                const int64_t v = (int64_t)c[j] + o[j];
-                inb = inb && v >= 0 && v < (int64_t)a.nCells[j];
-                dl += (int64_t)o[j] * a.mult[j];
-            }
-            if (inb) row(o, (uint64_t)((int64_t)rowBase + dl), originRow, false, 0u, 0u);
-            bool carry = true;
-#pragma unroll
-            for (int j = 1; j < K; j++) {
-                if (carry) {
-                    if (o[j] == 1) {
-                        o[j] = -1;
-                    } else {
-                        o[j]++;
-                        carry = false;
-                    }
-                }
-            }
+        for (int j = 1; j < K; j++) {
+            originRow = originRow && o[j] == 0;
+            const int64_t v = (int64_t)c[j] + o[j];
+            inb = inb && v >= 0 && v < (int64_t)a.nCells[j];
+            dl += (int64_t)o[j] * a.mult[j];
         }
-    } else {
-        // 3^(K-1) neighbour rows, 64 at a time: lane l looks up row b0 + l
-        // (its bounds and whether it can hold claimed candidates), then the
-        // wave visits the rows that can, in the same order as the odometer
-        // (o[1] fastest).  Rows left out are outside the grid, empty, or
-        // claimed by no lane: LID claims a row with every lane and cell iff
-        // its offset dl > 0 (|dl| >= nCells[0] off the origin row), Unicomp
-        // off the origin row by the parity of c[j] of its highest non-zero
-        // offset, the same for every lane.
-        for (int b0 = 0; b0 < nrow; b0 += 64) {
-            const int my = b0 + (int)lane;
-            int od[K];
-            od[0] = 0;
-            bool inb = my < nrow, org = true;
-            int64_t dl = 0;
-            int t = my;
+        if (inb) row(o, (uint64_t)((int64_t)rowBase + dl), originRow);
+        bool carry = true;
 #pragma unroll
-            for (int j = 1; j < K; j++) {
-                od[j] = t % 3 - 1;
-                t /= 3;
-                org = org && od[j] == 0;
-                const int64_t v = (int64_t)c[j] + od[j];
-                inb = inb && v >= 0 && v < (int64_t)a.nCells[j];
-                dl += (int64_t)od[j] * a.mult[j];
-            }
-            uint32_t r0 = 0u, r1 = 0u;
-            bool act = false;
-            if (inb) {
-                const uint64_t rbl = (uint64_t)((int64_t)rowBase + dl);
-                bool may = true;
-                if (a.form == SJ_FORM_LID) may = org || dl > 0;
-                else if (a.form == SJ_FORM_UNICOMP && !org) may = claims<K>(a.form, c, od, linA, rbl);
-                if (may) {
-                    r0 = pos_lb_t<DN>(a, rbl + ux0);
-                    r1 = pos_lb_t<DN>(a, rbl + ux1 + 1);
-                    act = r1 > r0;
+        for (int j = 1; j < K; j++) {
+            if (carry) {
+                if (o[j] == 1) {
+                    o[j] = -1;
+                } else {
+                    o[j]++;
+                    carry = false;
                 }
-            }
-            // the visited rows' offsets (2 bits per dim) and bases come from
-            // the lane that looked the row up
-            uint32_t opk = 0;
-#pragma unroll
-            for (int j = 1; j < K; j++) opk |= (uint32_t)(od[j] + 1) << (2 * (j - 1));
-            const uint64_t rbl = (uint64_t)((int64_t)rowBase + dl);
-            uint64_t am = __ballot(act);
-            while (am) {
-                const int bl = __builtin_ctzll(am);
-                am &= am - 1ull;
-                const uint32_t ok = readlane_u32(opk, bl);
-                int o[K];
-                o[0] = 0;
-                bool originRow = true;
-#pragma unroll
-                for (int j = 1; j < K; j++) {
-                    o[j] = (int)((ok >> (2 * (j - 1))) & 3u) - 1;
-                    originRow = originRow && o[j] == 0;
-                }
-                row(o, readlane_u64(rbl, bl), originRow, true, readlane_u32(r0, bl), readlane_u32(r1, bl));
             }
         }
     }
@@ -967,25 +810,13 @@ __device__ __forceinline__ void process_tile(const JoinArgs &a, uint32_t tile, L
     st.err += err;
 }
 
-template <int K, int D, int PASS, int PREC, bool RP, class LDS, bool DN = false>
-__device__ __forceinline__ void join_body(const JoinArgs &a, LDS *lds) {
-    if (PASS == PASS_FILL && !fill_gate(a)) return;
+// The waves of a launch over the tiles of a: run(tile) for each, from the
+// work queue or in cell order, then the statistics and the record's demand.
+template <int PASS, class Run>
+__device__ __forceinline__ void tile_loop(const JoinArgs &a, LaneStats &st, TileRec &R, Run run) {
     const unsigned wave = threadIdx.x >> 6;
     const unsigned lane = __lane_id();
-    LDS &L = lds[wave];
     const uint32_t nTiles = *a.nTilesDev;
-    LaneStats st;
-    TileRec R;
-    auto run = [&](uint32_t tile) __attribute__((always_inline)) {
-        if constexpr (RP) {
-            process_tile<K, D, PASS, PREC, true, LDS, DN>(a, tile, L, st, R);
-        } else if (D > 0 && a.useTiles) {
-            process_tile<K, D, PASS, PREC, false, LDS, DN>(a, tile, L, st, R);
-        } else {
-            const uint64_t s = (uint64_t)a.tileStart[tile] + lane;
-            if (s < a.tileStart[tile + 1]) process_point<K, D, PASS, PREC, DN>(a, (uint32_t)s, st);
-        }
-    };
     if (a.tileOrder) {
         // work queue in QSLICES interleaved slices with one counter each:
         // blocks are dealt to the XCDs round-robin, so a slice is served by
@@ -1010,16 +841,65 @@ __device__ __forceinline__ void join_body(const JoinArgs &a, LDS *lds) {
     flush_stats(a, st);
     // mask words this wave's pieces needed, plus its last partial block,
     // on the second word of the wave's counter slice
-    if (PASS == PASS_COUNT && a.recDir && lane == 0) {
+    if (PASS == PASS_COUNT && a.recCtr && lane == 0) {
         const uint32_t sl = (blockIdx.x * WPB + wave) % REC_NSLICE;
         atomicAdd(&a.recCtr[REC_SLICE0 + sl * REC_STRIDE + 1], (unsigned long long)(R.want + REC_BLK));
     }
 }
 
+template <int K, int D, int PASS, int PREC, bool RP, class LDS, bool DN = false>
+__device__ __forceinline__ void join_body(const JoinArgs &a, LDS *lds) {
+    if (PASS == PASS_FILL && !fill_gate(a)) return;
+    LDS &L = lds[threadIdx.x >> 6];
+    LaneStats st;
+    TileRec R;
+    tile_loop<PASS>(a, st, R, [&](uint32_t tile) __attribute__((always_inline)) {
+        if constexpr (RP) {
+            process_tile<K, D, PASS, PREC, true, LDS, DN>(a, tile, L, st, R);
+        } else {
+            if constexpr (D > 0 && K < SPAN_MINK) {
+                if (a.useTiles) {
+                    process_tile<K, D, PASS, PREC, false, LDS, DN>(a, tile, L, st, R);
+                    return;
+                }
+            }
+            const uint64_t s = (uint64_t)a.tileStart[tile] + __lane_id();
+            if (s < a.tileStart[tile + 1]) process_point<K, D, PASS, PREC, DN>(a, (uint32_t)s, st);
+        }
+    });
+}
+
+struct NoLds {};
+
+// d = k = 3 tile walk, and the per-point walk of the other shapes
 template <int K, int D, int PASS, int PREC>
 __global__ __launch_bounds__(JB) void k_join(JoinArgs a) {
-    __shared__ TileLds<D, PREC> lds[WPB];
+    __shared__ std::conditional_t<(D > 0 && K < SPAN_MINK), TileLds<D, PREC>, NoLds> lds[WPB];
     join_body<K, D, PASS, PREC, false>(a, lds);
+}
+
+// d = k >= 4: the span walk
+template <int K, int PASS, bool F32>
+__global__ __launch_bounds__(JB) __attribute__((amdgpu_waves_per_eu(F32 && K == 4 ? 4 : 3))) void k_span(JoinArgs a) {
+    __shared__ SpanLds lds[WPB];
+    if (PASS == PASS_FILL && !fill_gate(a)) return;
+    LaneStats st;
+    TileRec R;
+    tile_loop<PASS>(a, st, R, [&](uint32_t tile) __attribute__((always_inline)) {
+        process_span<K, PASS, F32>(a, tile, lds[threadIdx.x >> 6], st, R);
+    });
+}
+
+// and its fill from the record: no coordinates, one kernel for every k and
+// precision
+__global__ __launch_bounds__(JB) void k_span_rp(JoinArgs a) {
+    __shared__ SpanRows lds[WPB];
+    if (!fill_gate(a)) return;
+    LaneStats st;
+    TileRec R;
+    tile_loop<PASS_FILL>(a, st, R, [&](uint32_t tile) __attribute__((always_inline)) {
+        replay_span(a, tile, lds[threadIdx.x >> 6], st);
+    });
 }
 
 // k <= 2: four waves per SIMD (at most 128 VGPRs); measured faster at
@@ -1028,23 +908,6 @@ template <int K, int D, int PASS, int PREC, bool DN = false>
 __global__ __launch_bounds__(JB) __attribute__((amdgpu_waves_per_eu(4))) void k_join_o4(JoinArgs a) {
     __shared__ TileLds<D, PREC> lds[WPB];
     join_body<K, D, PASS, PREC, false, TileLds<D, PREC>, DN>(a, lds);
-}
-
-// 5 <= k <= 7: three waves per SIMD (at most 168 VGPRs), which the LDS
-// of these tiles still allows; measured faster at 6-D than the two waves
-// the compiler's own allocation leaves
-template <int K, int D, int PASS, int PREC, bool DN = false>
-__global__ __launch_bounds__(JB) __attribute__((amdgpu_waves_per_eu(3))) void k_join_o3(JoinArgs a) {
-    __shared__ TileLds<D, PREC> lds[WPB];
-    join_body<K, D, PASS, PREC, false, TileLds<D, PREC>, DN>(a, lds);
-}
-
-// 5 <= k <= 7, FP64 count: four waves per SIMD, which its registers (at
-// most 128) and the count-only LDS allow
-template <int K, int D, bool DN = false>
-__global__ __launch_bounds__(JB) __attribute__((amdgpu_waves_per_eu(4))) void k_join_c4(JoinArgs a) {
-    __shared__ TileLdsCount<D, 0> lds[WPB];
-    join_body<K, D, PASS_COUNT, 0, false, TileLdsCount<D, 0>, DN>(a, lds);
 }
 
 // Fill that replays the hit record of a count pass of precision PREC
@@ -1084,7 +947,7 @@ template <>
 struct LdsMax<0> {
     static constexpr int v = cmax<(int)sizeof(WideLds), (int)sizeof(MfmaLds<64>)>::v;
 };
-constexpr int MANY_LDS = (LdsMax<DEV_MAXK>::v + 15) / 16 * 16;
+constexpr int MANY_LDS = (cmax<LdsMax<SPAN_MINK - 1>::v, (int)sizeof(SpanLds)>::v + 15) / 16 * 16;
 // FP32 instances none of which uses the matrix cores: the FP32 LDS tile
 // walks only
 template <int D>
@@ -1096,12 +959,19 @@ template <>
 struct LdsMax32<0> {
     static constexpr int v = 0;
 };
-constexpr int MANY_LDS32 = (LdsMax32<DEV_MAXK>::v + 15) / 16 * 16;
+constexpr int MANY_LDS32 = (cmax<LdsMax32<SPAN_MINK - 1>::v, (int)sizeof(SpanLds)>::v + 15) / 16 * 16;
 
 template <int K, int PASS, int PREC, bool RP>
 __device__ __forceinline__ void many_tile(const JoinArgs &a, uint32_t tile, unsigned char *raw, LaneStats &st,
                                           TileRec &R) {
-    if constexpr (RP) {
+    if constexpr (K >= SPAN_MINK) {
+        // the wide walk (FP64 only) keeps no record
+        if (PREC == 1 || a.d == K) {
+            SpanLds &L = *reinterpret_cast<SpanLds *>(raw);
+            if constexpr (RP) replay_span(a, tile, L, st);
+            else process_span<K, PASS, PREC == 1>(a, tile, L, st, R);
+        } else process_tile_wide<PASS>(a, tile, *reinterpret_cast<WideLds *>(raw), st);
+    } else if constexpr (RP) {
         // the LDS tile walks replay their record; the wide walk keeps none
         if (PREC == 1) process_tile<K, K, PASS, 1, true>(a, tile, *reinterpret_cast<TileLdsIds<K, 1> *>(raw), st, R);
         else if (a.d == K) process_tile<K, K, PASS, 0, true>(a, tile, *reinterpret_cast<TileLdsIds<K, 0> *>(raw), st, R);
@@ -1198,7 +1068,7 @@ __device__ __forceinline__ void many_body(const JoinArgs *__restrict__ args, con
     if (cur != 0xFFFFFFFFu) {
         flush_stats(args[cur], st);
         // record words this wave's items needed (the record is shared)
-        if (PASS == PASS_COUNT && args[cur].recDir && lane == 0) {
+        if (PASS == PASS_COUNT && args[cur].recCtr && lane == 0) {
             const uint32_t sl = (blockIdx.x * WPB + wave) % REC_NSLICE;
             atomicAdd(&args[cur].recCtr[REC_SLICE0 + sl * REC_STRIDE + 1], (unsigned long long)(R.want + REC_BLK));
         }
@@ -1223,16 +1093,26 @@ __global__ __launch_bounds__(JB) __attribute__((amdgpu_waves_per_eu(3))) void k_
     many_body<PASS, 2, RP>(args, workInst, workTile, W, qctr, chunk, useQueue, &lds[0][0], MANY_LDS32);
 }
 
-// Tiles: runs of at most 64 consecutive points of one cell row within
-// [q0, q1).  A head starts every row and every 64 points inside a row.
-__global__ __launch_bounds__(JB) void k_tile_heads(JoinArgs a, uint32_t q0, uint32_t q1, uint32_t *head) {
+// Tiles: runs of at most 64 consecutive points of one cell row, or of one
+// cell group of the span walk, within [q0, q1).  A head starts every row (or
+// group) and every 64 points inside one.
+// pk (span walk): the cell coordinates modulo 4 per position, 4 bits per dim.
+__global__ __launch_bounds__(JB) void k_tile_heads(JoinArgs a, uint32_t q0, uint32_t q1, uint32_t *head,
+                                                   uint32_t *pk) {
     const uint64_t i = (uint64_t)blockIdx.x * JB + threadIdx.x;
     const uint64_t s = (uint64_t)q0 + i;
     if (s >= q1) return;
     const uint32_t cell = a.cellOf[s];
-    const uint64_t row = a.cellLinear[cell] - a.cellCoord[(uint64_t)cell * a.k];
+    uint64_t row = a.cellLinear[cell];
+    const int g = a.spanG > 0 ? a.spanG : 1;
+    for (int j = 0; j < g; j++) row -= (uint64_t)a.cellCoord[(uint64_t)cell * a.k + j] * (uint64_t)a.mult[j];
     const uint32_t rs = max(pos_lb(a, row), q0);
     head[i] = ((s - rs) & 63u) == 0 ? 1u : 0u;
+    if (pk) {
+        uint32_t v = 0;
+        for (int j = 0; j < a.k; j++) v |= (a.cellCoord[(uint64_t)cell * a.k + j] & 3u) << (4 * j);
+        pk[s] = v;
+    }
 }
 
 // z: counters of the join that follows, cleared here (each when set)
@@ -1245,6 +1125,7 @@ __global__ __launch_bounds__(JB) void k_tile_compact(const uint32_t *head, const
     if (z.mir && i < z.n) z.mir[i] = 0u;
     if (z.stat && i < 8) z.stat[i] = 0ull;
     if (z.qctr && i < (uint64_t)QSLICES * QSTRIDE) z.qctr[i] = 0u;
+    if (z.rec && i < REC_NCTR) z.rec[i] = 0ull;
     if (i >= len) return;
     if (head[i]) tileStart[ex[i]] = q0 + (uint32_t)i;
     if (i == len - 1) {
@@ -1326,63 +1207,58 @@ __device__ __forceinline__ uint32_t cost_key(uint32_t v) {
 constexpr uint32_t QB = 256;
 static_assert(JB == (int)QB, "one thread per class");
 
-// Tile cost: the candidates the tile stages, i.e. the union of its
-// neighbour cell ranges over the 3^(k-1) neighbour rows, as a class
-// (cost_key) per tile, counted per class in bucket[].
-template <int K>
-__global__ __launch_bounds__(JB) void k_tile_cost(JoinArgs a, uint32_t bound, uint32_t *key, uint32_t *bucket) {
+// Per tile, from its candidate ranges over the 3^(k-g) neighbour rows or
+// groups (g = 1 for rows): pieces, the bound of the pieces a walk executes
+// (sum of ceil(range / cw); chunks are whole multiples of cw), which lays out
+// the hit record once scanned; and the work-queue class (cost_key of the
+// candidates), counted per class in bucket[].  LPT lanes share a tile's
+// rows: one thread walking all 3^7 of them took 1.46 ms (bound) plus 1.27 ms
+// (cost) for 100,000 points in 8-D.
+template <int K, int LPT>
+__global__ __launch_bounds__(JB) void k_tile_ranges(JoinArgs a, uint32_t bound, uint32_t cw, uint32_t *pieces,
+                                                    uint32_t *key, uint32_t *bucket) {
     __shared__ uint32_t hist[QB];
     hist[threadIdx.x] = 0u;
     __syncthreads();
-    const uint32_t t = blockIdx.x * JB + threadIdx.x;
-    uint32_t cost = 0;
-    if (t < bound && t < *a.nTilesDev) {
-        const uint32_t s0 = a.tileStart[t], s1 = a.tileStart[t + 1] - 1u;
-        const uint32_t cA = a.cellOf[s0], cB = a.cellOf[s1];
+    const uint64_t gid = (uint64_t)blockIdx.x * JB + threadIdx.x;
+    const uint32_t t = (uint32_t)(gid / LPT);
+    const int sub = (int)(gid % LPT);
+    const bool live = t < bound && t < *a.nTilesDev;
+    uint32_t pc = 0, cost = 0;
+    if (live) {
+        const int g = a.spanG > 0 ? a.spanG : 1;
+        const uint32_t cA = a.cellOf[a.tileStart[t]], cB = a.cellOf[a.tileStart[t + 1] - 1u];
         uint32_t c[K];
 #pragma unroll
         for (int j = 0; j < K; j++) c[j] = a.cellCoord[(uint64_t)cA * K + j];
-        const uint32_t xb = a.cellCoord[(uint64_t)cB * K];
-        const uint64_t rowBase = a.cellLinear[cA] - c[0];
-        const uint32_t nC0 = a.nCells[0];
-        const uint32_t ux0 = c[0] >= 1 ? c[0] - 1 : 0u;
-        const uint32_t ux1 = xb + 1 < nC0 ? xb + 1 : nC0 - 1;
-        int o[K];
+        const TileSpan sp = tile_span<K>(a, g, c, a.cellLinear[cA], a.cellLinear[cB]);
+        int ng = 1;
 #pragma unroll
-        for (int j = 0; j < K; j++) o[j] = -1;
-        int nrow = 1;
-#pragma unroll
-        for (int j = 1; j < K; j++) nrow *= 3;
-        for (int it = 0; it < nrow; ++it) {
-            bool inb = true;
-            int64_t dl = 0;
-#pragma unroll
-            for (int j = 1; j < K; j++) {
-                const int64_t v = (int64_t)c[j] + o[j];
-                inb = inb && v >= 0 && v < (int64_t)a.nCells[j];
-                dl += (int64_t)o[j] * a.mult[j];
-            }
-            if (inb) {
-                const uint64_t rb = (uint64_t)((int64_t)rowBase + dl);
-                cost += pos_lb(a, rb + ux1 + 1) - pos_lb(a, rb + ux0);
-            }
-            bool carry = true;
-#pragma unroll
-            for (int j = 1; j < K; j++) {
-                if (carry) {
-                    if (o[j] == 1) {
-                        o[j] = -1;
-                    } else {
-                        o[j]++;
-                        carry = false;
-                    }
-                }
-            }
+        for (int j = 0; j < K; j++)
+            if (j >= g) ng *= 3;
+        for (int my = sub; my < ng; my += LPT) {
+            int od[K];
+            int64_t dl;
+            if (!span_group<K>(a, g, c, my, od, dl)) continue;
+            const uint32_t r = pos_lb(a, (uint64_t)((int64_t)sp.hi + dl)) - pos_lb(a, (uint64_t)((int64_t)sp.lo + dl));
+            pc += (r + cw - 1u) / cw;
+            cost += r;
         }
-        const uint32_t kk = cost_key(cost);
-        key[t] = kk;
-        atomicAdd(&hist[kk], 1u);
     }
+#pragma unroll
+    for (int off = LPT / 2; off > 0; off >>= 1) {
+        pc += __shfl_xor(pc, off, 64);
+        cost += __shfl_xor(cost, off, 64);
+    }
+    if (sub == 0) {
+        if (pieces && t < bound) pieces[t] = pc;
+        if (key && live) {
+            const uint32_t kk = cost_key(cost);
+            key[t] = kk;
+            atomicAdd(&hist[kk], 1u);
+        }
+    }
+    if (!bucket) return;
     __syncthreads();
     const uint32_t h = hist[threadIdx.x];
     if (h) atomicAdd(&bucket[threadIdx.x], h);
@@ -1444,27 +1320,6 @@ __global__ __launch_bounds__(JB) void k_tile_place(const uint32_t *nTilesDev, co
     }
     __syncthreads();
     if (valid) order[base[kk] + wcnt[wave][kk] + rank] = t;
-}
-
-// Pieces a tile walk may execute per tile (tile_piece_bound); zero
-// for entries from nTiles to bound.  Scanned, they lay out the hit record.
-template <int K>
-// zeroCtr (when set): the hit-record counters, cleared here
-__global__ __launch_bounds__(JB) void k_tile_bound(JoinArgs a, uint32_t bound, uint32_t cw, uint32_t *out,
-                                                   unsigned long long *zeroCtr) {
-    const uint32_t t = blockIdx.x * JB + threadIdx.x;
-    if (zeroCtr && t < REC_NCTR) zeroCtr[t] = 0ull;
-    if (t >= bound) return;
-    uint32_t v = 0;
-    if (t < *a.nTilesDev) {
-        const uint32_t cA = a.cellOf[a.tileStart[t]], cB = a.cellOf[a.tileStart[t + 1] - 1u];
-        uint32_t c[K];
-#pragma unroll
-        for (int j = 0; j < K; j++) c[j] = a.cellCoord[(uint64_t)cA * K + j];
-        const uint64_t rowBase = a.cellLinear[cA] - c[0];
-        v = tile_piece_bound<K>(a, c, rowBase, c[0], a.cellCoord[(uint64_t)cB * K], cw);
-    }
-    out[t] = v;
 }
 
 // ----------------------------------------------------- small row kernels
@@ -1579,9 +1434,6 @@ static JoinKernel pick_pass(int pass, int prec) {
     if constexpr (K <= 2 && D > 0) {
         if (pass == PASS_COUNT) return prec ? k_join_o4<K, D, PASS_COUNT, 1> : k_join_o4<K, D, PASS_COUNT, 0>;
         return prec ? k_join_o4<K, D, PASS_FILL, 1> : k_join_o4<K, D, PASS_FILL, 0>;
-    } else if constexpr (K >= 5 && K <= 7 && D > 0) {
-        if (pass == PASS_COUNT) return prec ? k_join_o3<K, D, PASS_COUNT, 1> : k_join_c4<K, D>;
-        return prec ? k_join_o3<K, D, PASS_FILL, 1> : k_join_o3<K, D, PASS_FILL, 0>;
     } else {
         if (pass == PASS_COUNT) return prec ? k_join<K, D, PASS_COUNT, 1> : k_join<K, D, PASS_COUNT, 0>;
         return prec ? k_join<K, D, PASS_FILL, 1> : k_join<K, D, PASS_FILL, 0>;
@@ -1642,32 +1494,37 @@ static WorkKernel pick_workload(int k) {
     return nullptr;
 }
 
-using TileCostKernel = void (*)(JoinArgs, uint32_t, uint32_t *, uint32_t *);
-static TileCostKernel pick_tile_cost(int k) {
+using TileRangesKernel = void (*)(JoinArgs, uint32_t, uint32_t, uint32_t *, uint32_t *, uint32_t *);
+// lanes per tile: about its number of neighbour rows, 64 at most
+static TileRangesKernel pick_tile_ranges(int k, unsigned *lanes) {
+    *lanes = k == 1 ? 1 : (k == 2 ? 4 : (k == 3 ? 16 : 64));
     switch (k) {
-    case 1: return k_tile_cost<1>;
-    case 2: return k_tile_cost<2>;
-    case 3: return k_tile_cost<3>;
-    case 4: return k_tile_cost<4>;
-    case 5: return k_tile_cost<5>;
-    case 6: return k_tile_cost<6>;
-    case 7: return k_tile_cost<7>;
-    case 8: return k_tile_cost<8>;
+    case 1: return k_tile_ranges<1, 1>;
+    case 2: return k_tile_ranges<2, 4>;
+    case 3: return k_tile_ranges<3, 16>;
+    case 4: return k_tile_ranges<4, 64>;
+    case 5: return k_tile_ranges<5, 64>;
+    case 6: return k_tile_ranges<6, 64>;
+    case 7: return k_tile_ranges<7, 64>;
+    case 8: return k_tile_ranges<8, 64>;
     }
     return nullptr;
 }
 
-using TileBoundKernel = void (*)(JoinArgs, uint32_t, uint32_t, uint32_t *, unsigned long long *);
-static TileBoundKernel pick_tile_bound(int k) {
+template <int K>
+static JoinKernel pick_span_k(int pass, int prec) {
+    if (pass == PASS_COUNT) return prec ? k_span<K, PASS_COUNT, true> : k_span<K, PASS_COUNT, false>;
+    return prec ? k_span<K, PASS_FILL, true> : k_span<K, PASS_FILL, false>;
+}
+
+static JoinKernel pick_span(int k, int pass, int prec, bool replay) {
+    if (replay) return k_span_rp;
     switch (k) {
-    case 1: return k_tile_bound<1>;
-    case 2: return k_tile_bound<2>;
-    case 3: return k_tile_bound<3>;
-    case 4: return k_tile_bound<4>;
-    case 5: return k_tile_bound<5>;
-    case 6: return k_tile_bound<6>;
-    case 7: return k_tile_bound<7>;
-    case 8: return k_tile_bound<8>;
+    case 4: return pick_span_k<4>(pass, prec);
+    case 5: return pick_span_k<5>(pass, prec);
+    case 6: return pick_span_k<6>(pass, prec);
+    case 7: return pick_span_k<7>(pass, prec);
+    case 8: return pick_span_k<8>(pass, prec);
     }
     return nullptr;
 }
@@ -1758,7 +1615,111 @@ JoinArgs base_args(sj_grid_s *g, int form, double T) {
     a.qEnd = (uint32_t)g->n;
     a.wBegin = 0;
     a.wEnd = (uint32_t)g->n;
+    a.nPts = (uint32_t)g->n;
     return a;
+}
+
+// Dims g of a span-walk group, by the expected time per point.  With rho
+// points per occupied cell and e_j occupied cells per dim, a group of dims
+// < g holds G = rho * prod_{j<g} e_j points in about G / 64 + 1/2 tiles; a tile
+// meets prod_{j>=g} (3 - 2 / e_j) groups in the grid, and in each of them its
+// own cells plus 2 M cells (M: the cells one step of every dim < g spans), at
+// most the group.  A small g leaves tiles half empty and meets many short
+// ranges, a large one takes candidates that are far away.
+// Measured in 8-D (100,000 points): this rule's group of more dims takes 17%
+// more pairs than the next smaller one and is faster, 1.22 against 1.49 ms.
+static int choose_span(const sj_grid_s *g) {
+    const int k = g->k;
+    const double rho = (double)g->n / (double)std::max<uint64_t>(1, g->nNonEmpty);
+    double e[DEV_MAXK], box = 1.0;
+    for (int j = 0; j < k; j++) {
+        e[j] = std::max(1.0, (double)g->gp.nCells[j] - 2.0);  // the grid is one cell wider on both sides
+        box *= e[j];
+    }
+    // the share of the cells that is occupied, spread evenly over the dims
+    const double share = std::pow(std::min(1.0, (double)g->nNonEmpty / box), 1.0 / k);
+    for (int j = 0; j < k; j++) e[j] = std::max(1.0, e[j] * share);
+    // cycles per candidate of a tile (matrix instructions, threshold,
+    // compares) and per range
+    const double evalCy = (k > 4 ? 32.0 : 16.0) + 12.0, rangeCy = 600.0;
+    int best = 1;
+    double bestCost = INFINITY, cells = 1.0, M = 0.0;
+    for (int gd = 1; gd <= k; gd++) {
+        M += cells;
+        cells *= e[gd - 1];
+        double groups = 1.0;
+        for (int j = gd; j < k; j++) groups *= 3.0 - 2.0 / e[j];
+        const double G = std::max(1.0, rho * cells);
+        const double lanes = G / (G / 64.0 + 0.5);
+        const double span = std::min(cells, lanes / rho + 2.0 * M) * rho;
+        const double cost = groups * (span * evalCy + rangeCy) / lanes;
+        if (cost < bestCost) {
+            bestCost = cost;
+            best = gd;
+        }
+    }
+    return best;
+}
+
+// Constants of the span filter in precision u (2^-24 or 2^-53), KP the dims
+// padded to the matrix instruction (4 or 8).  With y = x - centre rounded to
+// the precision (the FP64 difference is rounded once, and again to FP32), a
+// vector is off by at most 1.0001 u |y| (1.01 * 2^-53 |y| in FP64), so the pair's
+// squared distance moves by at most 4.01 u s, s = |q|^2 + |c|^2 of the rounded
+// vectors.  Norms err by at most KP u s, their scaling by 2 u s, the
+// accumulation of KP products onto the norm by (KP + 2) u times its terms
+// (at most 2 s), the lane's threshold by u (s + T): (3 KP + 11) u s + u T in
+// all, to first order.  alpha = 1.1 (3 KP + 16) u covers it, so a pair whose
+// true squared distance is at most T' passes at the threshold T' (1 + 8 u);
+// the canonical sum accepts true squared distances up to
+// T' = T / (1 - 1.01 (k + 3) 2^-53).  tiny covers denormals flushed in the
+// matrix cores.
+struct SpanBand {
+    double scale, T1;
+};
+static SpanBand span_band(double T, int k, bool f32) {
+    const double u = std::ldexp(1.0, f32 ? -24 : -53);
+    const int KP = (k + 3) / 4 * 4;
+    SpanBand b;
+    b.scale = 1.0 - 1.1 * (3 * KP + 16) * u;
+    const double rho = 1.01 * (k + 3) * std::ldexp(1.0, -53), tiny = KP * std::ldexp(1.0, f32 ? -118 : -1000);
+    b.T1 = T / (1.0 - rho) * (1.0 + 8.0 * u) + tiny;
+    if (f32) {
+        // both used as floats: away from the hit side
+        float f = (float)b.scale;
+        if ((double)f > b.scale) f = std::nextafter(f, 0.0f);
+        b.scale = f;
+        f = (float)b.T1;
+        if ((double)f < b.T1) f = std::nextafter(f, INFINITY);
+        b.T1 = f;
+    }
+    return b;
+}
+
+sj_status span_setup(sj_grid_s *g, JoinArgs &a, int prec) {
+    a.spanG = 0;
+    if (!a.useTiles || g->d != g->k || g->k < SPAN_MINK || g->k > DEV_MAXK) return SJ_OK;
+    const bool f32 = prec == SJ_PREC_FP32_RECHECK;
+    a.spanG = choose_span(g);
+    double R = 0.0;
+    for (int j = 0; j < g->k; j++) R = std::max(R, g->gp.maxArr[j] - g->gp.minArr[j]);
+    // squares of differences stay far from overflow, T far from underflow
+    a.spanDirect = f32 ? !(R < 1e15 && a.T > 1e-30) : !(R < 1e140 && a.T > 1e-280);
+    const SpanBand b = span_band(a.T, g->k, f32);
+    a.spanScale = b.scale;
+    a.spanT1 = b.T1;
+    SJ_TRY(g->posPk.alloc(&g->ctx->pool, g->n));
+    a.posPk = g->posPk.p;
+    return SJ_OK;
+}
+
+// Upper bound of the tiles over len points: one per 64 points plus one per
+// cell row or group with points.
+static uint64_t tile_count_bound(const sj_grid_s *g, const JoinArgs &a, uint64_t len) {
+    uint64_t groups = std::min<uint64_t>(len, g->nNonEmpty);
+    uint64_t all = 1;
+    for (int j = a.spanG > 0 ? a.spanG : 1; j < g->k && all <= groups; j++) all *= g->gp.nCells[j];
+    return (len + 63) / 64 + std::min(groups, all);
 }
 
 static sj_status cell_workload(sj_grid_s *g, int lid, DBuf<uint32_t> &w) {
@@ -1787,36 +1748,14 @@ sj_status build_tiles(sj_grid_s *g, const JoinArgs &a, uint32_t q0, uint32_t q1,
         SJ_TRY(fill_u32(s, nTiles.p, 1, 0u));
         return SJ_OK;
     }
-    hipLaunchKernelGGL(k_tile_heads, dim3(nblk(len)), dim3(JB), 0, s, a, q0, q1, head.p);
+    hipLaunchKernelGGL(k_tile_heads, dim3(nblk(len)), dim3(JB), 0, s, a, q0, q1, head.p,
+                       a.spanG > 0 ? g->posPk.p : nullptr);
     SJ_LAUNCH_CHECK();
     SJ_TRY(scan_exclusive_u32_to_u32(pool, s, head.p, len, ex.p));
-    const uint64_t nz = std::max<uint64_t>(len, std::max<uint64_t>(2 * QB, std::max<uint64_t>(zero.n, 256)));
+    uint64_t nz = std::max<uint64_t>(len, std::max<uint64_t>(2 * QB, std::max<uint64_t>(zero.n, 256)));
+    if (zero.rec) nz = std::max<uint64_t>(nz, REC_NCTR);
     hipLaunchKernelGGL(k_tile_compact, dim3(nblk(nz)), dim3(JB), 0, s, head.p, ex.p, q0, q1, tileStart.p, nTiles.p,
                        zero);
-    SJ_LAUNCH_CHECK();
-    return SJ_OK;
-}
-
-// Work queue: tiles by descending staged-candidate bucket.  The tile count
-// stays on the device: the sort covers an upper bound (one tile per 64
-// points plus one per non-empty row, at most one per non-empty cell).
-static sj_status build_tile_queue(sj_grid_s *g, const JoinArgs &a, uint64_t len, DBuf<uint32_t> &order,
-                                  uint32_t *classes) {
-    Pool *pool = &g->ctx->pool;
-    hipStream_t s = g->ctx->stream;
-    const uint64_t bound64 = (len + 63) / 64 + std::min<uint64_t>(len, g->nNonEmpty);
-    if (bound64 > 0xFFFFFFFFull) {
-        set_error("work queue: %llu tiles exceed 32-bit indices", (unsigned long long)bound64);
-        return SJ_ERR_OVERFLOW;
-    }
-    const uint32_t bound = (uint32_t)bound64;
-    DBuf<uint32_t> key;
-    SJ_TRY(key.alloc(pool, bound));
-    SJ_TRY(order.alloc(pool, bound));
-    if (bound == 0) return SJ_OK;
-    hipLaunchKernelGGL(pick_tile_cost(g->k), dim3(nblk(bound)), dim3(JB), 0, s, a, bound, key.p, classes);
-    SJ_LAUNCH_CHECK();
-    hipLaunchKernelGGL(k_tile_place, dim3(nblk(bound)), dim3(JB), 0, s, a.nTilesDev, key.p, classes, order.p);
     SJ_LAUNCH_CHECK();
     return SJ_OK;
 }
@@ -1864,18 +1803,11 @@ static JoinKernel pick_replay_k(int prec) {
     else return prec ? k_join_rp<K, K, 1> : k_join_rp<K, K, 0>;
 }
 
-// k = d = 2 or 6 on a dense grid: kernels without the binary-search
-// lookups (the 2-D and 6-D shapes; other k use the general kernels)
-static JoinKernel pick_dense(int k, int pass, int prec, bool replay) {
-    if (k == 2) {
-        if (replay) return prec ? k_join_rp_o5<2, 2, 1, true> : k_join_rp_o5<2, 2, 0, true>;
-        if (pass == PASS_COUNT)
-            return prec ? k_join_o4<2, 2, PASS_COUNT, 1, true> : k_join_o4<2, 2, PASS_COUNT, 0, true>;
-        return prec ? k_join_o4<2, 2, PASS_FILL, 1, true> : k_join_o4<2, 2, PASS_FILL, 0, true>;
-    }
-    if (replay) return prec ? k_join_rp<6, 6, 1, true> : k_join_rp<6, 6, 0, true>;
-    if (pass == PASS_COUNT) return prec ? k_join_o3<6, 6, PASS_COUNT, 1, true> : k_join_c4<6, 6, true>;
-    return prec ? k_join_o3<6, 6, PASS_FILL, 1, true> : k_join_o3<6, 6, PASS_FILL, 0, true>;
+// k = d = 2 on a dense grid: kernels without the binary-search lookups
+static JoinKernel pick_dense2(int pass, int prec, bool replay) {
+    if (replay) return prec ? k_join_rp_o5<2, 2, 1, true> : k_join_rp_o5<2, 2, 0, true>;
+    if (pass == PASS_COUNT) return prec ? k_join_o4<2, 2, PASS_COUNT, 1, true> : k_join_o4<2, 2, PASS_COUNT, 0, true>;
+    return prec ? k_join_o4<2, 2, PASS_FILL, 1, true> : k_join_o4<2, 2, PASS_FILL, 0, true>;
 }
 
 static JoinKernel pick_replay(int k, int prec) {
@@ -1883,11 +1815,6 @@ static JoinKernel pick_replay(int k, int prec) {
     case 1: return pick_replay_k<1>(prec);
     case 2: return pick_replay_k<2>(prec);
     case 3: return pick_replay_k<3>(prec);
-    case 4: return pick_replay_k<4>(prec);
-    case 5: return pick_replay_k<5>(prec);
-    case 6: return pick_replay_k<6>(prec);
-    case 7: return pick_replay_k<7>(prec);
-    case 8: return pick_replay_k<8>(prec);
     }
     return nullptr;
 }
@@ -1908,8 +1835,10 @@ static sj_status launch_join(sj_grid_s *g, const JoinArgs &a, int pass, int prec
     if (prec == SJ_PREC_FP32_RECHECK && a.mDP > 0) return launch_join_mfma(a, pass, g->ctx->cu_count, s, replay);
     if (prec == SJ_PREC_FP64 && a.useTiles && wide_supported(g->d, g->k))
         return launch_join_wide(a, pass, g->ctx->cu_count, s);
-    JoinKernel kfn = replay ? pick_replay(g->k, prec) : pick_kernel(g->k, g->d, pass, prec);
-    if (a.posLB && g->k == g->d && (g->k == 2 || g->k == 6)) kfn = pick_dense(g->k, pass, prec, replay);
+    JoinKernel kfn;
+    if (a.spanG > 0) kfn = pick_span(g->k, pass, prec, replay);
+    else if (a.posLB && g->k == g->d && g->k == 2) kfn = pick_dense2(pass, prec, replay);
+    else kfn = replay ? pick_replay(g->k, prec) : pick_kernel(g->k, g->d, pass, prec);
     if (!kfn) {
         set_error("no traversal kernel for k=%d", g->k);
         return SJ_ERR_UNSUPPORTED;
@@ -1944,26 +1873,16 @@ sj_status launch_join_many(const JoinArgs *d_args, const uint32_t *workInst, con
     return SJ_OK;
 }
 
-sj_status launch_tile_bound(const JoinArgs &a, int k, uint32_t bound, uint32_t cw, uint32_t *out, hipStream_t s) {
-    TileBoundKernel kfn = pick_tile_bound(k);
+sj_status launch_tile_ranges(const JoinArgs &a, int k, uint32_t bound, uint32_t cw, uint32_t *pieces, uint32_t *key,
+                             uint32_t *bucket, hipStream_t s) {
+    unsigned lanes = 1;
+    TileRangesKernel kfn = pick_tile_ranges(k, &lanes);
     if (!kfn) {
-        set_error("tile bound: k=%d above the device stencil limit", k);
+        set_error("tile ranges: k=%d above the device stencil limit", k);
         return SJ_ERR_UNSUPPORTED;
     }
     if (bound == 0) return SJ_OK;
-    hipLaunchKernelGGL(kfn, dim3((bound + JB - 1) / JB), dim3(JB), 0, s, a, bound, cw, out, nullptr);
-    SJ_LAUNCH_CHECK();
-    return SJ_OK;
-}
-
-sj_status launch_tile_cost(const JoinArgs &a, int k, uint32_t bound, uint32_t *key, uint32_t *val, hipStream_t s) {
-    TileCostKernel kfn = pick_tile_cost(k);
-    if (!kfn) {
-        set_error("tile cost: k=%d above the device stencil limit", k);
-        return SJ_ERR_UNSUPPORTED;
-    }
-    if (bound == 0) return SJ_OK;
-    hipLaunchKernelGGL(kfn, dim3((bound + JB - 1) / JB), dim3(JB), 0, s, a, bound, key, val);
+    hipLaunchKernelGGL(kfn, dim3(nblk((uint64_t)bound * lanes)), dim3(JB), 0, s, a, bound, cw, pieces, key, bucket);
     SJ_LAUNCH_CHECK();
     return SJ_OK;
 }
@@ -2201,7 +2120,37 @@ sj_status join(sj_grid_s *g, const sj_join_params *P, sj_result_s *r) {
         SJ_TRY(qclass.alloc(pool, 2 * QB));
         SJ_TRY(qctr.alloc(pool, QSLICES * QSTRIDE));
     }
-    const TileZero tz{queue ? qclass.p : nullptr, mir.p, n, stat, queue ? qctr.p : nullptr};
+    SJ_TRY(span_setup(g, a, prec));
+    const uint64_t tBound = tile_count_bound(g, a, n);
+    if (tBound > 0xFFFFFFFFull) {
+        set_error("join: %llu tiles exceed 32-bit indices", (unsigned long long)tBound);
+        return SJ_ERR_OVERFLOW;
+    }
+    // hit record of the count pass for the fill, in space that persists
+    // on the context; without the space the fill evaluates distances again.
+    // The span walk's record needs no directory.
+    DBuf<uint64_t> recDir, recMask, tileDir, recStart;
+    DBuf<uint32_t> tileBound, recN, qkey;
+    DBuf<unsigned long long> recCtr;
+    const bool span = a.spanG > 0;
+    bool recording = P->hit_record >= 0 && record_walk(g, a) && n > 0;
+    uint64_t dirCap = 0, maskCap = 0;
+    if (recording) {
+        dirCap = span ? 0 : std::max<uint64_t>(ctx->recDirCap, std::max<uint64_t>(1ull << 20, n));
+        maskCap = std::max<uint64_t>(ctx->recMaskCap, std::max<uint64_t>(1ull << 23, 16 * n));
+        bool room = recMask.alloc(pool, maskCap) == SJ_OK && recCtr.alloc(pool, REC_NCTR) == SJ_OK;
+        if (span)
+            room = room && recStart.alloc(pool, tBound) == SJ_OK && recN.alloc(pool, tBound) == SJ_OK;
+        else
+            room = room && recDir.alloc(pool, (uint64_t)REC_DW * dirCap) == SJ_OK &&
+                   tileDir.alloc(pool, tBound + 1) == SJ_OK && tileBound.alloc(pool, tBound) == SJ_OK;
+        if (!room) {
+            recording = false;  // no room: the fill evaluates distances again
+            (void)hipGetLastError();
+        }
+    }
+    const TileZero tz{queue ? qclass.p : nullptr, mir.p, n, stat, queue ? qctr.p : nullptr,
+                      recording ? recCtr.p : nullptr};
     SJ_TRY(build_tiles(g, a, 0u, (uint32_t)n, tileStart, nTilesDev, tz));
     a.tileStart = tileStart.p;
     a.nTilesDev = nTilesDev.p;
@@ -2210,39 +2159,34 @@ sj_status join(sj_grid_s *g, const sj_join_params *P, sj_result_s *r) {
     a.ownCnt = own.p;
     a.mirCnt = mir.p;
     a.stat = stat;
-    // hit record of the count pass for the fill, in space that persists
-    // on the context; without the space the fill evaluates distances again
-    DBuf<uint64_t> recDir, recMask, tileDir;
-    DBuf<uint32_t> tileBound;
-    DBuf<unsigned long long> recCtr;
-    bool recording = P->hit_record >= 0 && record_walk(g, a) && n > 0;
-    const uint64_t tBound = (n + 63) / 64 + std::min<uint64_t>(n, g->nNonEmpty);
+    // one launch for the record's layout and the queue's classes
+    const uint32_t cw = a.mDP > 0 ? 32u : 64u;  // candidates per recorded piece
+    const bool dir = recording && !span;
+    if (queue) {
+        SJ_TRY(qkey.alloc(pool, tBound));
+        SJ_TRY(tileOrder.alloc(pool, tBound));
+        tw.start();
+    }
+    if (queue || dir)
+        SJ_TRY(launch_tile_ranges(a, g->k, (uint32_t)tBound, cw, dir ? tileBound.p : nullptr,
+                                  queue ? qkey.p : nullptr, queue ? qclass.p : nullptr, s));
+    if (dir) SJ_TRY(scan_exclusive_u32_to_u64(pool, s, tileBound.p, tBound, tileDir.p));
     if (recording) {
-        const uint64_t dirCap = std::max<uint64_t>(ctx->recDirCap, std::max<uint64_t>(1ull << 20, n));
-        const uint64_t maskCap = std::max<uint64_t>(ctx->recMaskCap, std::max<uint64_t>(1ull << 23, 16 * n));
-        if (tBound > 0xFFFFFFFFull || recDir.alloc(pool, (uint64_t)REC_DW * dirCap) != SJ_OK ||
-            recMask.alloc(pool, maskCap) != SJ_OK || tileDir.alloc(pool, tBound + 1) != SJ_OK ||
-            tileBound.alloc(pool, tBound) != SJ_OK || recCtr.alloc(pool, REC_NCTR) != SJ_OK) {
-            recording = false;  // no room: the fill evaluates distances again
-            (void)hipGetLastError();
-        } else {
-            const uint32_t cw = a.mDP > 0 ? 32u : 64u;  // candidates per recorded piece
-            // the record's counters cleared by the same launch
-            hipLaunchKernelGGL(pick_tile_bound(g->k), dim3(nblk(std::max<uint64_t>(tBound, REC_NCTR))), dim3(JB), 0,
-                               s, a, (uint32_t)tBound, cw, tileBound.p, recCtr.p);
-            SJ_LAUNCH_CHECK();
-            SJ_TRY(scan_exclusive_u32_to_u64(pool, s, tileBound.p, tBound, tileDir.p));
-            a.recDir = recDir.p;
-            a.recMask = recMask.p;
-            a.tileDir = tileDir.p;
-            a.recCtr = recCtr.p;
-            a.dirCap = dirCap;
-            a.maskCap = maskCap;
-        }
+        a.recDir = recDir.p;
+        a.recMask = recMask.p;
+        a.tileDir = tileDir.p;
+        a.recN = recN.p;
+        a.recStart = recStart.p;
+        a.recCtr = recCtr.p;
+        a.dirCap = dirCap;
+        a.maskCap = maskCap;
     }
     if (queue) {
-        tw.start();
-        SJ_TRY(build_tile_queue(g, a, n, tileOrder, qclass.p));
+        if (tBound) {
+            hipLaunchKernelGGL(k_tile_place, dim3(nblk(tBound)), dim3(JB), 0, s, a.nTilesDev, qkey.p, qclass.p,
+                               tileOrder.p);
+            SJ_LAUNCH_CHECK();
+        }
         tw.stop();
         a.tileOrder = tileOrder.p;
         a.qctr = qctr.p;
@@ -2272,7 +2216,7 @@ sj_status join(sj_grid_s *g, const sj_join_params *P, sj_result_s *r) {
     // again only if the result outgrew the buffer.
     uint64_t *pin = ctx->pinned;
     const CountScalars csc{r->d_offsets.p + n, stat, recording ? recCtr.p : nullptr,
-                           recording ? tileDir.p + tBound : nullptr, scal.p};
+                           dir ? tileDir.p + tBound : nullptr, scal.p};
     const bool ahead = P->capacity == 0 && !r->extIds && ctx->idsHint > 0;
     // ahead: the fill's first cursor kernel gathers them
     if (!ahead) {
@@ -2542,6 +2486,8 @@ sj_status join(sj_grid_s *g, const sj_join_params *P, sj_result_s *r) {
             ab.tileOrder = nullptr;  // batches walk their tiles in order
             ab.tileStart = tileStart.p + t0;
             ab.tileDir = a.tileDir ? a.tileDir + t0 : nullptr;
+            ab.recN = a.recN ? a.recN + t0 : nullptr;
+            ab.recStart = a.recStart ? a.recStart + t0 : nullptr;
             ab.nTilesDev = bCount[sl].p;
             ab.qBegin = hTile.p[t0];
             ab.qEnd = hTile.p[t1];

@@ -105,8 +105,8 @@ struct sj_many_s {
     // hit record shared by the instances: the count kernel records, the fill
     // kernel replays (the wide walk's instances evaluate again)
     bool rec = false;
-    DBuf<uint32_t> tBound;
-    DBuf<uint64_t> tileDir, recDir, recMask;
+    DBuf<uint32_t> tBound, recN;
+    DBuf<uint64_t> tileDir, recDir, recMask, recStart;
     DBuf<unsigned long long> recCtr;
     uint64_t dirCap = 0, maskCap = 0;
 
@@ -316,6 +316,7 @@ sj_status plan(sj_many_s *m, const sj_instance *in, int count) {
             a.pts32 = nullptr;
             a.mDP = 0;
         }
+        SJ_TRY(span_setup(I.g, a, P.precision));
         SJ_TRY(build_tiles(I.g, a, 0u, (uint32_t)x.n, I.tileStart, I.nTilesDev));
         a.tileStart = I.tileStart.p;
         a.nTilesDev = I.nTilesDev.p;
@@ -397,7 +398,8 @@ sj_status plan(sj_many_s *m, const sj_instance *in, int count) {
         SJ_TRY(val2.alloc(pool, W));
         uint64_t w0 = 0;
         for (int i = 0; i < count; i++) {
-            SJ_TRY(launch_tile_cost(m->args[i], m->args[i].k, m->inst[i].nTiles, key.p + w0, val.p + w0, s));
+            SJ_TRY(launch_tile_ranges(m->args[i], m->args[i].k, m->inst[i].nTiles, 64u, nullptr, key.p + w0, nullptr,
+                                      s));
             w0 += m->inst[i].nTiles;
         }
         hipLaunchKernelGGL(k_iota_u32, dim3(nb(W)), dim3(JB), 0, s, val.p, (uint64_t)W);
@@ -415,10 +417,16 @@ sj_status plan(sj_many_s *m, const sj_instance *in, int count) {
     if (P.hit_record >= 0 && W) {
         SJ_TRY(m->tBound.alloc(pool, W));
         SJ_TRY(m->tileDir.alloc(pool, (uint64_t)W + 1));
+        SJ_TRY(m->recN.alloc(pool, W));
+        SJ_TRY(m->recStart.alloc(pool, W));
         uint64_t w0 = 0;
         for (int i = 0; i < count; i++) {
             const uint32_t cw = m->args[i].mDP > 0 ? 32u : 64u;
-            SJ_TRY(launch_tile_bound(m->args[i], m->args[i].k, m->inst[i].nTiles, cw, m->tBound.p + w0, s));
+            if (m->args[i].spanG > 0)  // its record has no directory
+                SJ_TRY(fill_u32(s, m->tBound.p + w0, m->inst[i].nTiles, 0u));
+            else
+                SJ_TRY(launch_tile_ranges(m->args[i], m->args[i].k, m->inst[i].nTiles, cw, m->tBound.p + w0, nullptr,
+                                          nullptr, s));
             w0 += m->inst[i].nTiles;
         }
         SJ_TRY(scan_exclusive_u32_to_u64(pool, s, m->tBound.p, W, m->tileDir.p));
@@ -434,6 +442,8 @@ sj_status plan(sj_many_s *m, const sj_instance *in, int count) {
             a.recDir = m->recDir.p;
             a.recMask = m->recMask.p;
             a.tileDir = m->tileDir.p + w0;
+            a.recN = m->recN.p + w0;
+            a.recStart = m->recStart.p + w0;
             a.recCtr = m->recCtr.p;
             a.dirCap = m->dirCap;
             a.maskCap = m->maskCap;

@@ -69,6 +69,15 @@ struct JoinArgs {
     const uint64_t *tileDir;       // tile t: entries [tileDir[t], tileDir[t+1])
     unsigned long long *recCtr;    // REC_* counters
     uint64_t dirCap, maskCap;      // entries, words
+    // span walk (spanG > 0): tiles are runs of points of one group of cells
+    // with the same coordinates in dims spanG..k-1 (spanG = 0: one cell row)
+    int spanG;
+    uint32_t nPts;             // points in the sorted arrays
+    int spanDirect;            // no filter: the predicate for every candidate
+    double spanScale, spanT1;  // filter: norms scaled by 1 - alpha, threshold
+    const uint32_t *posPk;     // per point: cell coordinates modulo 4, 4 bits per dim
+    uint32_t *recN;            // record words per tile
+    uint64_t *recStart;        // and the first of them
 };
 
 // Hit-record counters: record unusable (any cause), then REC_NSLICE
@@ -552,6 +561,7 @@ struct TileZero {
     uint64_t n = 0;
     unsigned long long *stat = nullptr;
     uint32_t *qctr = nullptr;
+    unsigned long long *rec = nullptr;  // hit-record counters
 };
 sj_status build_tiles(sj_grid_s *g, const JoinArgs &a, uint32_t q0, uint32_t q1, DBuf<uint32_t> &tileStart,
                       DBuf<uint32_t> &nTiles, const TileZero &zero = TileZero{});
@@ -564,13 +574,15 @@ sj_status prepare_fp32(sj_grid_s *g, JoinArgs &a, int *prec);
 sj_status launch_join_many(const JoinArgs *d_args, const uint32_t *workInst, const uint32_t *workTile,
                            uint32_t W, uint32_t *qctr, uint32_t chunk, int useQueue, int pass, int mfma,
                            unsigned blocks, hipStream_t s, bool replay = false);
-// Per-tile bound of the pieces a walk executes (cw candidates per piece)
-// for the first `bound` tiles of a.
-sj_status launch_tile_bound(const JoinArgs &a, int k, uint32_t bound, uint32_t cw, uint32_t *out, hipStream_t s);
+// Per tile of the first `bound` tiles of a (each output when set): pieces, a
+// bound of the pieces of cw candidates a walk executes (zero past the last
+// tile); key, the work-queue class (descending 8-bit log-scale bucket of the
+// candidates), counted per class in bucket[].
+sj_status launch_tile_ranges(const JoinArgs &a, int k, uint32_t bound, uint32_t cw, uint32_t *pieces, uint32_t *key,
+                             uint32_t *bucket, hipStream_t s);
 
-// Work-queue keys of tiles [0, bound) of one join (descending 8-bit
-// log-scale bucket of the staged candidates; val[t] = t).
-sj_status launch_tile_cost(const JoinArgs &a, int k, uint32_t bound, uint32_t *key, uint32_t *val, hipStream_t s);
+// Chooses the span walk for joins with d = k >= 4 and sets its fields.
+sj_status span_setup(sj_grid_s *g, JoinArgs &a, int prec);
 
 // Plain FP64 traversal from LDS-staged candidates for d != k or d > 8, d <= 64.
 bool wide_supported(int d, int k);

@@ -46,6 +46,19 @@ struct MfmaLds {
     float nq[64];         // squared norms of the tile's queries
 };
 
+// Sum of v over groups of G consecutive lanes (G = 1, 2, 4, 8 or 16, aligned),
+// in every lane: DPP moves only.  Once the lanes of a half agree, its mirror
+// image is the other half's sum.
+template <int G>
+__device__ __forceinline__ float group_sum(float v) {
+    auto add = [](float x, int y) __attribute__((always_inline)) { return x + __int_as_float(y); };
+    if constexpr (G >= 2) v = add(v, __builtin_amdgcn_mov_dpp(__float_as_int(v), 0xB1, 0xF, 0xF, true));
+    if constexpr (G >= 4) v = add(v, __builtin_amdgcn_mov_dpp(__float_as_int(v), 0x4E, 0xF, 0xF, true));
+    if constexpr (G >= 8) v = add(v, __builtin_amdgcn_mov_dpp(__float_as_int(v), 0x141, 0xF, 0xF, true));
+    if constexpr (G >= 16) v = add(v, __builtin_amdgcn_mov_dpp(__float_as_int(v), 0x140, 0xF, 0xF, true));
+    return v;
+}
+
 // RP (fill only): take each chunk's hit masks from the count pass's hit
 // record (one directory entry per executed 32-candidate chunk) instead of
 // the matrix cores; chunks without hits are skipped.
@@ -191,6 +204,25 @@ __device__ __forceinline__ void process_tile_mfma(const JoinArgs &a, uint32_t ti
                 if (PASS == PASS_COUNT && valid)
                     cand += (useL ? e1 - e0 : 0) + (useC ? e2 - e1 : 0) + (useR ? e3 - e2 : 0);
                 const bool mirC = anyMirror && !originRow;
+                // FP32 copy: a chunk's rows are loaded all together, and
+                // while the chunk before is on the matrix cores.  Loaded one
+                // after another at the start of their chunk they cost 132 ms
+                // instead of 98 ms at 500,000 points in 64-D (matrix
+                // instructions alone: 42 ms).
+                constexpr int NV = DP >= 8 ? DP / 8 : 1;  // float4 per lane and chunk
+                float4 pre[RP ? 1 : NV];
+                uint32_t have = 0xFFFFFFFFu;  // the chunk in pre
+                auto fetch = [&](uint32_t c0) __attribute__((always_inline)) {
+                    if constexpr (!RP) {
+#pragma unroll
+                        for (int i = 0; i < NV; i++) {
+                            const uint32_t f = lane + 64u * (uint32_t)i;
+                            const uint32_t t = min(c0 + f / (DP / 4), u1 - 1u);  // past the row: its norm says so
+                            pre[i] = *reinterpret_cast<const float4 *>(P32 + (uint64_t)t * DP + f % (DP / 4) * 4);
+                        }
+                        have = c0;
+                    }
+                };
                 for (uint32_t cb = u0; cb < u1; cb += 32) {
                     const uint32_t nv = min(32u, u1 - cb);
                     if (PASS == PASS_FILL && !anyOwnW && (cb + nv <= a.wBegin || cb >= a.wEnd)) {
@@ -224,25 +256,26 @@ __device__ __forceinline__ void process_tile_mfma(const JoinArgs &a, uint32_t ti
                     if (src32) {
                         // float4 f of the chunk goes to lane f % 64; the DP/4
                         // lanes of a candidate are consecutive, so its norm is
-                        // a shuffle reduction
-                        for (uint32_t f = lane; f < 8u * DP; f += 64) {
+                        // a group sum
+                        if (have != cb) fetch(cb);
+#pragma unroll
+                        for (int i = 0; i < NV; i++) {
+                            const uint32_t f = lane + 64u * (uint32_t)i;
                             const uint32_t cj = f / (DP / 4), part = f % (DP / 4);
-                            float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
-                            if (cj < nv) {
-                                const float4 w =
-                                    *reinterpret_cast<const float4 *>(P32 + (uint64_t)(cb + cj) * DP + part * 4);
-                                const float4 cc = *reinterpret_cast<const float4 *>(&L.ctr32[part * 4]);
-                                v = make_float4(w.x - cc.x, w.y - cc.y, w.z - cc.z, w.w - cc.w);
-                            }
-                            *reinterpret_cast<float4 *>(&L.x[cj][part * 4]) = v;
+                            const float4 w = pre[i];
+                            const float4 cc = *reinterpret_cast<const float4 *>(&L.ctr32[part * 4]);
+                            const float4 v = make_float4(w.x - cc.x, w.y - cc.y, w.z - cc.z, w.w - cc.w);
                             float nn = v.x * v.x;
                             nn = fmaf(v.y, v.y, nn);
                             nn = fmaf(v.z, v.z, nn);
                             nn = fmaf(v.w, v.w, nn);
-#pragma unroll
-                            for (int off = DP / 8; off > 0; off >>= 1) nn += __shfl_xor(nn, off, 64);
-                            if (part == 0) L.nc[cj] = cj < nv ? nn : 1e30f;
+                            nn = group_sum<DP / 4>(nn);
+                            if (DP >= 8 || cj < 32u) {  // 4 padded dims: 32 lanes hold the chunk
+                                *reinterpret_cast<float4 *>(&L.x[cj][part * 4]) = v;
+                                if (part == 0) L.nc[cj] = cj < nv ? nn : 1e30f;
+                            }
                         }
+                        if (cb + 32u < u1) fetch(cb + 32u);
                         if (lane < 32) {
                             L.id[lane] = lane < nv ? (int32_t)a.origId[cb + lane] : -1;
                             L.cnt[lane] = 0u;
@@ -301,10 +334,10 @@ __device__ __forceinline__ void process_tile_mfma(const JoinArgs &a, uint32_t ti
                     // the masks of query q over the 32 candidates: ballot
                     // (h, r) carries queries q0 (low word) and q0 + 4 (high
                     // word) with q0 = 32h + 8(r/4) + r%4, whose bit 2 is 0
+                    // Few registers hold a pair near eps: the others end
+                    // after one compare
                     uint32_t myM = 0, myS = 0, myL = 0;
                     bool anyM = false;
-                    const unsigned laneQ = lane & ~4u;
-                    const bool laneHi = (lane & 4u) != 0u;
 #pragma unroll
                     for (int h = 0; h < 2; h++) {
 #pragma unroll
@@ -314,16 +347,20 @@ __device__ __forceinline__ void process_tile_mfma(const JoinArgs &a, uint32_t ti
                             const float dot = h == 0 ? acc0[r] : acc1[r];
                             const float d2 = fmaf(-2.0f, dot, sq);
                             const float M = fmaf(a.mAlpha, sq, a.mBeta);
-                            const uint64_t bm = __ballot(d2 - M <= a.mThi);
-                            const uint64_t bs = __ballot(d2 + M <= a.mTlo);
-                            const bool mine = laneQ == (unsigned)(32 * h + 8 * (r / 4) + (r % 4));
-                            myM = mine ? (laneHi ? (uint32_t)(bm >> 32) : (uint32_t)bm) : myM;
-                            myS = mine ? (laneHi ? (uint32_t)(bs >> 32) : (uint32_t)bs) : myS;
+                            const uint64_t bm = __builtin_amdgcn_ballot_w64(d2 - M <= a.mThi);
+                            if (bm == 0ull) continue;
+                            anyM = true;
+                            const uint64_t bs = __builtin_amdgcn_ballot_w64(d2 + M <= a.mTlo);
+                            unsigned q = lane;  // opaque: the lane masks are not kept through the walk
+                            asm volatile("" : "+v"(q));
+                            const bool mine = (q & ~4u) == (unsigned)(32 * h + 8 * (r / 4) + (r % 4));
+                            const bool hi = (q & 4u) != 0u;
+                            myM = mine ? (hi ? (uint32_t)(bm >> 32) : (uint32_t)bm) : myM;
+                            myS = mine ? (hi ? (uint32_t)(bs >> 32) : (uint32_t)bs) : myS;
                             if (PASS == PASS_COUNT) {
-                                const uint64_t bl = __ballot(d2 <= a.mT32);
-                                myL = mine ? (laneHi ? (uint32_t)(bl >> 32) : (uint32_t)bl) : myL;
+                                const uint64_t bl = __builtin_amdgcn_ballot_w64(d2 <= a.mT32);
+                                myL = mine ? (hi ? (uint32_t)(bl >> 32) : (uint32_t)bl) : myL;
                             }
-                            anyM = anyM || bm != 0ull;
                         }
                     }
                     uint32_t hitRec = 0;  // the chunk's final hits, for the record

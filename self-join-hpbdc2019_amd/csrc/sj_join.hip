@@ -970,16 +970,16 @@ __device__ __forceinline__ void many_tile(const JoinArgs &a, uint32_t tile, unsi
             SpanLds &L = *reinterpret_cast<SpanLds *>(raw);
             if constexpr (RP) replay_span(a, tile, L, st);
             else process_span<K, PASS, PREC == 1>(a, tile, L, st, R);
-        } else process_tile_wide<PASS>(a, tile, *reinterpret_cast<WideLds *>(raw), st);
+        } else process_tile_wide<PASS>(a, tile, *reinterpret_cast<WideLds *>(raw), st, R);
     } else if constexpr (RP) {
         // the LDS tile walks replay their record; the wide walk keeps none
         if (PREC == 1) process_tile<K, K, PASS, 1, true>(a, tile, *reinterpret_cast<TileLdsIds<K, 1> *>(raw), st, R);
         else if (a.d == K) process_tile<K, K, PASS, 0, true>(a, tile, *reinterpret_cast<TileLdsIds<K, 0> *>(raw), st, R);
-        else process_tile_wide<PASS>(a, tile, *reinterpret_cast<WideLds *>(raw), st);
+        else process_tile_wide<PASS>(a, tile, *reinterpret_cast<WideLds *>(raw), st, R);
     } else {
         if (PREC == 1) process_tile<K, K, PASS, 1, false>(a, tile, *reinterpret_cast<TileLds<K, 1> *>(raw), st, R);
         else if (a.d == K) process_tile<K, K, PASS, 0, false>(a, tile, *reinterpret_cast<TileLds<K, 0> *>(raw), st, R);
-        else process_tile_wide<PASS>(a, tile, *reinterpret_cast<WideLds *>(raw), st);
+        else process_tile_wide<PASS>(a, tile, *reinterpret_cast<WideLds *>(raw), st, R);
     }
 }
 
@@ -1843,9 +1843,13 @@ static JoinKernel pick_replay(int k, int prec) {
 }
 
 // Walks whose count pass keeps a hit record the fill can replay: the LDS
-// tile walk (d = k <= 8) and the matrix-core walk (FP32, mDP > 0).
-static bool record_walk(const sj_grid_s *g, const JoinArgs &a) {
-    return a.useTiles && ((g->d == g->k && g->d <= DEV_MAXK) || a.mDP > 0);
+// tile walk and the span walk (d = k <= 8), the matrix-core walk (FP32,
+// mDP > 0) and the wide walk (FP64, same record).
+static bool wide_walk(const sj_grid_s *g, const JoinArgs &a, int prec) {
+    return prec == SJ_PREC_FP64 && a.useTiles && wide_supported(g->d, g->k);
+}
+static bool record_walk(const sj_grid_s *g, const JoinArgs &a, int prec) {
+    return a.useTiles && ((g->d == g->k && g->d <= DEV_MAXK) || a.mDP > 0 || wide_walk(g, a, prec));
 }
 
 sj_status tpp_point_order(sj_grid_s *g, const uint32_t *corder, DBuf<uint32_t> &order);
@@ -1856,8 +1860,15 @@ static sj_status launch_join(sj_grid_s *g, const JoinArgs &a, int pass, int prec
     hipStream_t s = g->ctx->stream;
     if (a.tppOrder) return launch_join_tpp(a, g->k, pass, g->n, s);
     if (prec == SJ_PREC_FP32_RECHECK && a.mDP > 0) return launch_join_mfma(a, pass, g->ctx->cu_count, s, replay);
-    if (prec == SJ_PREC_FP64 && a.useTiles && wide_supported(g->d, g->k))
-        return launch_join_wide(a, pass, g->ctx->cu_count, s);
+    if (wide_walk(g, a, prec)) {
+        if (!replay) return launch_join_wide(a, pass, g->ctx->cu_count, s);
+        // the matrix-core walk's replay touches no coordinates: at any width
+        // (evaluating again cost as much as the count: 5.1 ms at 60,000
+        // points in 17-D)
+        JoinArgs ar = a;
+        ar.mDP = 4;
+        return launch_join_mfma(ar, pass, g->ctx->cu_count, s, true);
+    }
     JoinKernel kfn;
     if (a.spanG > 0) kfn = pick_span(g->k, pass, prec, replay);
     else if (a.posLB && g->k == g->d && g->k == 2) kfn = pick_dense2(pass, prec, replay);
@@ -2155,8 +2166,9 @@ sj_status join(sj_grid_s *g, const sj_join_params *P, sj_result_s *r) {
     DBuf<uint64_t> recDir, recMask, tileDir, recStart;
     DBuf<uint32_t> tileBound, recN, qkey;
     DBuf<unsigned long long> recCtr;
-    const bool span = a.spanG > 0;
-    bool recording = P->hit_record >= 0 && record_walk(g, a) && n > 0;
+    const bool span = a.spanG > 0, wide = wide_walk(g, a, prec);
+    const bool slots = a.mDP == 0 && !wide;  // the record holds the mirrored hits' slots
+    bool recording = P->hit_record >= 0 && record_walk(g, a, prec) && n > 0;
     uint64_t dirCap = 0, maskCap = 0;
     if (recording) {
         dirCap = span ? 0 : std::max<uint64_t>(ctx->recDirCap, std::max<uint64_t>(1ull << 20, n));
@@ -2183,7 +2195,7 @@ sj_status join(sj_grid_s *g, const sj_join_params *P, sj_result_s *r) {
     a.mirCnt = mir.p;
     a.stat = stat;
     // one launch for the record's layout and the queue's classes
-    const uint32_t cw = a.mDP > 0 ? 32u : 64u;  // candidates per recorded piece
+    const uint32_t cw = a.mDP > 0 || wide ? 32u : 64u;  // candidates per recorded piece
     const bool dir = recording && !span;
     if (queue) {
         SJ_TRY(qkey.alloc(pool, tBound));
@@ -2321,7 +2333,7 @@ sj_status join(sj_grid_s *g, const sj_join_params *P, sj_result_s *r) {
         CountScalars gsc = csc;
         if (!gather) gsc.out = nullptr;
         if (!gate) {
-            if (!(replay && a.mDP == 0)) {
+            if (!(replay && slots)) {
                 hipLaunchKernelGGL(k_mir_cursors, dim3(nbq), dim3(JB), 0, s, r->d_offsets.p, own.p, 0u,
                                    (uint32_t)n, 0ull, mirCur.p, nullptr, qz, gsc);
                 SJ_LAUNCH_CHECK();
@@ -2335,7 +2347,7 @@ sj_status join(sj_grid_s *g, const sj_join_params *P, sj_result_s *r) {
             SJ_TRY(launch_join(g, a, PASS_FILL, prec, replay));
         } else {
             hipLaunchKernelGGL(k_mir_cursors, dim3(nbq), dim3(JB), 0, s, r->d_offsets.p, own.p, 0u,
-                               (uint32_t)n, 0ull, mirCur.p, a.mDP == 0 ? recCtr.p + REC_BAD : nullptr, qz, gsc);
+                               (uint32_t)n, 0ull, mirCur.p, slots ? recCtr.p + REC_BAD : nullptr, qz, gsc);
             SJ_LAUNCH_CHECK();
             // replay when the record is usable; an unusable one (the
             // record's space fell short, seen on the host afterwards) is
@@ -2499,7 +2511,7 @@ sj_status join(sj_grid_s *g, const sj_join_params *P, sj_result_s *r) {
             const uint32_t t0 = (uint32_t)(std::upper_bound(hTile.p, hTile.p + nT + 1, (uint32_t)q0) - hTile.p) - 1u;
             const uint32_t t1 = (uint32_t)(std::lower_bound(hTile.p, hTile.p + nT + 1, (uint32_t)q1) - hTile.p);
             const uint64_t base = hOff.p[s0];
-            if (!(replay && a.mDP == 0)) {  // recorded slots need no cursors
+            if (!(replay && slots)) {  // recorded slots need no cursors
                 hipLaunchKernelGGL(k_mir_cursors, dim3(nblk(s1 - s0)), dim3(JB), 0, s, r->d_offsets.p, own.p, s0, s1,
                                    (unsigned long long)base, mirCur.p, nullptr, nullptr, CountScalars{});
                 SJ_LAUNCH_CHECK();

@@ -13,6 +13,7 @@ __global__ __launch_bounds__(JB) void k_join_wide(JoinArgs a) {
     WideLds &L = lds[wave];
     const uint32_t nTiles = *a.nTilesDev;
     LaneStats st;
+    TileRec R;
     if (a.tileOrder) {
         const uint32_t ns = min(gridDim.x, (uint32_t)QSLICES);
         const uint32_t sl = blockIdx.x % ns;
@@ -23,14 +24,19 @@ __global__ __launch_bounds__(JB) void k_join_wide(JoinArgs a) {
             if (q >= nTiles) break;
             uint32_t nx = 0;
             if (lane == 0) nx = atomicAdd(a.qctr + sl * QSTRIDE, 1u);
-            process_tile_wide<PASS>(a, a.tileOrder[q], L, st);
+            process_tile_wide<PASS, true>(a, a.tileOrder[q], L, st, R);
             i = (uint64_t)nbl * WPB + readlane_u32(nx, 0);
         }
     } else {
         for (uint32_t tile = blockIdx.x * WPB + wave; tile < nTiles; tile += gridDim.x * WPB)
-            process_tile_wide<PASS>(a, tile, L, st);
+            process_tile_wide<PASS, true>(a, tile, L, st, R);
     }
     flush_stats(a, st);
+    // record words this wave's chunks needed, plus its last partial block
+    if (PASS == PASS_COUNT && a.recCtr && lane == 0) {
+        const uint32_t sl = (blockIdx.x * WPB + wave) % REC_NSLICE;
+        atomicAdd(&a.recCtr[REC_SLICE0 + sl * REC_STRIDE + 1], (unsigned long long)(R.want + REC_BLK));
+    }
 }
 
 // Every grid the K == D tile walk does not cover, up to WIDE_MAXD dims.

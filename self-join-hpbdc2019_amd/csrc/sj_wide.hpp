@@ -29,8 +29,12 @@ struct WideLds {
     unsigned long long base[WIDE_CH];
 };
 
-template <int PASS>
-__device__ __forceinline__ void process_tile_wide(const JoinArgs &a, uint32_t tile, WideLds &L, LaneStats &st) {
+// REC (count): the hits of every chunk go into the hit record, one directory
+// entry per 32-candidate chunk as in the matrix-core walk, whose replaying
+// fill reads it.
+template <int PASS, bool REC = false>
+__device__ __forceinline__ void process_tile_wide(const JoinArgs &a, uint32_t tile, WideLds &L, LaneStats &st,
+                                                  TileRec &R) {
     const unsigned lane = __lane_id();
     const int k = a.k, d = a.d;
     const uint32_t ts0 = a.tileStart[tile], ts1 = a.tileStart[tile + 1];
@@ -54,6 +58,15 @@ __device__ __forceinline__ void process_tile_wide(const JoinArgs &a, uint32_t ti
     const uint32_t nC0 = a.nCells[0];
     const uint32_t x = c[0];
     const double *qp = a.pts + (uint64_t)sEff * d;
+    const bool recOn = REC && PASS == PASS_COUNT && a.recDir != nullptr;
+    bool rec = false;
+    uint64_t dbase = 0, dend = 0, piece_it = 0;
+    if (recOn) {
+        dbase = readlane_u64(a.tileDir[tile], 0);
+        dend = readlane_u64(a.tileDir[tile + 1], 0);
+        rec = dend <= a.dirCap && !badTile;
+        if (!rec && lane == 0) atomicAdd(&a.recCtr[REC_BAD], 1ull);
+    }
 
     const bool ownW = valid && s >= a.wBegin && s < a.wEnd;
     const int32_t myId = valid ? (int32_t)a.origId[s] : 0;
@@ -173,6 +186,8 @@ __device__ __forceinline__ void process_tile_wide(const JoinArgs &a, uint32_t ti
                     }
                     emit_chunk32<PASS>(a, cb, nv, hit, mirBits, ownW, myId, ownPos, ownLim, own, L.id, L.cnt,
                                        L.base, anyMirror, err);
+                    if (recOn) record_piece(a, R, rec, dbase, dend, piece_it, (uint64_t)hit);
+                    piece_it++;
                     wave_lds_sync();
                 }
             }

@@ -261,17 +261,19 @@ struct SpanQuery {
 
 // Room for n <= 64 more record words of the tile in progress (started: it
 // has words already): the first goes to the returned word, those from room
-// on to the next block.  False when the record space is exhausted.
+// on to the next block.  False when the record space is exhausted: the
+// wave's block then may lie past the space (rec_room of an earlier tile of
+// another instance), so not even a word that would fit in it is placed.
 __device__ __forceinline__ bool span_rec_room(const JoinArgs &a, TileRec &R, uint32_t n, bool started, uint64_t &at,
                                               uint32_t &room, uint64_t &next) {
     room = R.used < SPAN_LINK ? SPAN_LINK - R.used : 0u;
     at = R.blk + R.used;
     next = 0;
+    if (!R.ok) return false;
     if (n <= room) {
         R.used += n;
         return true;
     }
-    if (!R.ok) return false;
     const uint32_t sl = (blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6)) % REC_NSLICE;
     uint64_t b = 0;
     if (__lane_id() == 0) b = atomicAdd(&a.recCtr[REC_SLICE0 + sl * REC_STRIDE], 1ull);

@@ -1,0 +1,45 @@
+"""A batch of joins of different walks whose common hit record outgrows its
+first space while the plan sizes it: waves that failed to get a record block
+in one instance go on with tiles of another.  Every instance equals the
+oracle, after the plan and after a replay."""
+import numpy as np
+import pytest
+
+import oracle as O
+from sjamd import datasets as D
+
+pytestmark = pytest.mark.gpu
+
+# (dims, points, eps): the first instance alone fills the record's first
+# space, then come 2-D tiles (masks) and 4-D tiles (words per hit)
+SPEC = [(4, 250_000, 0.095), (2, 300_000, 0.006), (4, 200_000, 0.06)]
+
+_refs = {}
+
+
+def _batch():
+    if not _refs:
+        for i, (d, n, eps) in enumerate(SPEC):
+            pts = D.uniform(n, d, 70 + i)
+            _refs[i] = (pts, d, eps, O.join(pts, d, eps, O.LID, sort_rows=True))
+    return [_refs[i] for i in range(len(SPEC))]
+
+
+@pytest.mark.parametrize("schedule", [0, 1])
+@pytest.mark.parametrize("precision", [0, 1])
+def test_record_outgrown_across_walks(ctx, precision, schedule):
+    b = _batch()
+    N = sum(n for _, n, _ in SPEC)
+    # the full stencil records one word per ordered pair in 4-D
+    assert int(b[0][3][0][-1]) > max(1 << 23, 16 * N)
+    print(f"[many record] precision={precision} schedule={schedule}", flush=True)
+    m = ctx.many([(p, k, e) for p, k, e, _ in b], form="full", precision=precision, schedule=schedule)
+    for rep in range(2):
+        for i, (_, _, _, (roff, rids)) in enumerate(b):
+            off, ids = m.csr(i)
+            off, ids = O.csr_rows_sorted(np.asarray(off, dtype=np.uint64), np.asarray(ids, dtype=np.int32))
+            np.testing.assert_array_equal(off, roff, err_msg=f"replay {rep} instance {i}")
+            np.testing.assert_array_equal(ids, rids, err_msg=f"replay {rep} instance {i}")
+        if rep == 0:
+            m.run()
+    m.free()

@@ -29,8 +29,11 @@
 // predicate; the candidate in a cell adjacent to the query's (the span holds
 // cells further away, and the grid join leaves such pairs out even when
 // rounding puts their distance at eps); the form's claim.  Cells are compared
-// by their coordinates modulo 4 (posPk, 4 bits per dim): a pair within eps
-// lies at most two cells apart.
+// by their coordinates modulo 4 (posPk, 4 bits per dim): a pair that passes
+// the filter lies at most two cells apart, since a grid has fewer than 2^32
+// cells per dim and eps is far above underflow.  Under spanDirect neither
+// holds for the predicate (the squares of several eps may underflow to 0),
+// so there the coordinates themselves are compared.
 //
 // Hit record: one word per hit, candidate | query << 32 | mirrored slot << 38 |
 // (no mirrored hit) << 63, in the order of the walk, so a row's own hits keep ascending positions.  A
@@ -344,6 +347,12 @@ __device__ __forceinline__ void span_flush(const JoinArgs &a, SpanLds &L, uint32
     const uint32_t z = pk_diff(a.posPk[c], pkA);
     const bool same = c >= cs0 && c < cs1;  // the query's own cell
     bool ok = lane < nh && !pk_far(z);
+    if (a.spanDirect) {
+        const uint32_t *cc = a.cellCoord + (uint64_t)a.cellOf[c] * K;
+        const uint32_t *cq = a.cellCoord + (uint64_t)a.cellOf[ts0 + q] * K;
+#pragma unroll
+        for (int j = 0; j < K; j++) ok = ok && cc[j] - cq[j] + 1u <= 2u;
+    }
     if (a.form == SJ_FORM_LID) {
         ok = ok && c >= cs0;
     } else if (a.form != SJ_FORM_FULL) {

@@ -318,6 +318,15 @@ SJ_API int32_t sj_fp32_band(double T, double R, int32_t D, float *lo, float *hi,
  * Returns the padded operand width (4..64), 0 when d is above 64. */
 SJ_API int32_t sj_mfma_band(double T, double R, int32_t d, float *alpha, float *beta, float *tlo, float *thi);
 
+/* Filter of the walk for d = k = 4..8 (no reference counterpart).  With y = x
+ * minus the tile's first point, rounded to the precision (FP64, or FP32 for
+ * SJ_PREC_FP32_RECHECK), and all sums in that precision in any order, a pair
+ * with d2_64 <= T has |q|^2 scale - 2 q.c <= t1 - |c|^2 scale; pairs that pass
+ * are decided in FP64.  R bounds the differences of coordinates in a dim.
+ * Returns 1 when the filter is used, 0 when its range does not hold T and R
+ * (the join then evaluates the predicate for every candidate). */
+SJ_API int32_t sj_span_band(double T, double R, int32_t k, int32_t precision, double *scale, double *t1);
+
 #ifdef __cplusplus
 }
 #endif

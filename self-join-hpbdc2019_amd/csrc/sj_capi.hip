@@ -103,6 +103,13 @@ SJ_API int32_t sj_mfma_band(double T, double R, int32_t d, float *alpha, float *
     return b.DP;
 }
 
+SJ_API int32_t sj_span_band(double T, double R, int32_t k, int32_t precision, double *scale, double *t1) {
+    const SpanBand b = span_band(T, R, k, precision == SJ_PREC_FP32_RECHECK);
+    if (scale) *scale = b.scale;
+    if (t1) *t1 = b.T1;
+    return b.usable ? 1 : 0;
+}
+
 SJ_API sj_status sj_context_create(int32_t device, void *stream, sj_context *out) {
     if (!out) {
         set_error("sj_context_create: null output");

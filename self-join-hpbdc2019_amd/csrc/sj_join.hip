@@ -1685,7 +1685,8 @@ static int choose_span(const sj_grid_s *g) {
 }
 
 // Constants of the span filter in precision u (2^-24 or 2^-53), KP the dims
-// padded to the matrix instruction (4 or 8).  With y = x - centre rounded to
+// padded to the matrix instruction (4 or 8), for coordinates whose differences
+// are at most R.  With y = x - centre rounded to
 // the precision (the FP64 difference is rounded once, and again to FP32), a
 // vector is off by at most 1.0001 u |y| (1.01 * 2^-53 |y| in FP64), so the pair's
 // squared distance moves by at most 4.01 u s, s = |q|^2 + |c|^2 of the rounded
@@ -1697,13 +1698,14 @@ static int choose_span(const sj_grid_s *g) {
 // the canonical sum accepts true squared distances up to
 // T' = T / (1 - 1.01 (k + 3) 2^-53).  tiny covers denormals flushed in the
 // matrix cores.
-struct SpanBand {
-    double scale, T1;
-};
-static SpanBand span_band(double T, int k, bool f32) {
+// usable: squares of differences stay far from overflow, T far from underflow
+// (and from overflow: a grid's R is at least 2 eps, and the threshold must be
+// finite to reject the infinite norms of queries past the tile's end).
+SpanBand span_band(double T, double R, int k, bool f32) {
     const double u = std::ldexp(1.0, f32 ? -24 : -53);
     const int KP = (k + 3) / 4 * 4;
     SpanBand b;
+    b.usable = f32 ? R < 1e15 && T > 1e-30 : R < 1e140 && T > 1e-280;
     b.scale = 1.0 - 1.1 * (3 * KP + 16) * u;
     const double rho = 1.01 * (k + 3) * std::ldexp(1.0, -53), tiny = KP * std::ldexp(1.0, f32 ? -118 : -1000);
     b.T1 = T / (1.0 - rho) * (1.0 + 8.0 * u) + tiny;
@@ -1722,13 +1724,11 @@ static SpanBand span_band(double T, int k, bool f32) {
 sj_status span_setup(sj_grid_s *g, JoinArgs &a, int prec) {
     a.spanG = 0;
     if (!a.useTiles || g->d != g->k || g->k < SPAN_MINK || g->k > DEV_MAXK) return SJ_OK;
-    const bool f32 = prec == SJ_PREC_FP32_RECHECK;
     a.spanG = choose_span(g);
     double R = 0.0;
     for (int j = 0; j < g->k; j++) R = std::max(R, g->gp.maxArr[j] - g->gp.minArr[j]);
-    // squares of differences stay far from overflow, T far from underflow
-    a.spanDirect = f32 ? !(R < 1e15 && a.T > 1e-30) : !(R < 1e140 && a.T > 1e-280);
-    const SpanBand b = span_band(a.T, g->k, f32);
+    const SpanBand b = span_band(a.T, R, g->k, prec == SJ_PREC_FP32_RECHECK);
+    a.spanDirect = !b.usable;
     a.spanScale = b.scale;
     a.spanT1 = b.T1;
     SJ_TRY(g->posPk.alloc(&g->ctx->pool, g->n));

@@ -581,6 +581,14 @@ sj_status launch_join_many(const JoinArgs *d_args, const uint32_t *workInst, con
 sj_status launch_tile_ranges(const JoinArgs &a, int k, uint32_t bound, uint32_t cw, uint32_t *pieces, uint32_t *key,
                              uint32_t *bucket, hipStream_t s);
 
+// Filter of the span walk for k dims, threshold T and differences of
+// coordinates up to R: norms times scale, threshold T1; not usable: the walk
+// evaluates the predicate for every candidate (derivation in sj_join.hip).
+struct SpanBand {
+    double scale, T1;
+    bool usable;
+};
+SpanBand span_band(double T, double R, int k, bool f32);
 // Chooses the span walk for joins with d = k >= 4 and sets its fields.
 sj_status span_setup(sj_grid_s *g, JoinArgs &a, int prec);
 

@@ -110,7 +110,7 @@ EXPORTS = [
     "sj_batch_estimate", "sj_batch_estimate_workqueue", "sj_import_csv", "sj_sort_in_nd_bins", "sj_free_host", "sj_eps_threshold",
     "sj_many_create", "sj_many_run", "sj_many_autotune", "sj_many_set_tuning", "sj_many_get_tuning",
     "sj_many_instance", "sj_many_stats", "sj_many_times", "sj_many_count", "sj_many_free",
-    "sj_fp32_band", "sj_mfma_band",
+    "sj_fp32_band", "sj_mfma_band", "sj_span_band",
     "sj_self_join_static", "sj_static_need", "sj_static_scratch_bytes",
 ]
 
@@ -135,6 +135,8 @@ def lib():
     L.sj_fp32_band.argtypes = [C.c_double, C.c_double, i32, fp, fp, fp]
     L.sj_mfma_band.restype = i32
     L.sj_mfma_band.argtypes = [C.c_double, C.c_double, i32, fp, fp, fp, fp]
+    L.sj_span_band.restype = i32
+    L.sj_span_band.argtypes = [C.c_double, C.c_double, i32, i32, P(C.c_double), P(C.c_double)]
     L.sj_context_create.argtypes = [i32, vp, P(vp)]
     L.sj_context_destroy.argtypes = [vp]
     L.sj_context_destroy.restype = None
@@ -214,6 +216,13 @@ def mfma_band(T, R, d):
     v = [C.c_float() for _ in range(4)]
     dp = lib().sj_mfma_band(float(T), float(R), int(d), *[C.byref(x) for x in v])
     return (dp,) + tuple(x.value for x in v)
+
+
+def span_band(T, R, k, precision):
+    """(usable, scale, T1) of the filter of the walk for d = k = 4..8."""
+    scale, t1 = C.c_double(), C.c_double()
+    u = lib().sj_span_band(float(T), float(R), int(k), int(precision), C.byref(scale), C.byref(t1))
+    return bool(u), scale.value, t1.value
 
 
 _hip_rt = None

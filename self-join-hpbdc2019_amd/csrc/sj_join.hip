@@ -1762,11 +1762,12 @@ sj_status build_tiles(sj_grid_s *g, const JoinArgs &a, uint32_t q0, uint32_t q1,
     Pool *pool = &g->ctx->pool;
     hipStream_t s = g->ctx->stream;
     const uint64_t len = q1 - q0;
+    // what stays is allocated first: an arena gets the rest back at the end
+    SJ_TRY(tileStart.alloc(pool, len + 1));
+    SJ_TRY(nTiles.alloc(pool, 1));
     DBuf<uint32_t> head, ex;
     SJ_TRY(head.alloc(pool, len));
     SJ_TRY(ex.alloc(pool, len + 1));
-    SJ_TRY(tileStart.alloc(pool, len + 1));
-    SJ_TRY(nTiles.alloc(pool, 1));
     if (len == 0) {
         SJ_TRY(fill_u32(s, nTiles.p, 1, 0u));
         return SJ_OK;

@@ -36,7 +36,10 @@ bool g_done[MAX_DEVICES] = {};
 // (join_need) draw from the pool for n points, every buffer counted as if
 // none were released and padded to 256 bytes: the input check of the entry
 // point.  The dense lookup table is not counted: it is built only when it
-// fits beside the join's share.
+// fits beside the join's share.  Nor are the cell keys of d = k >= 4 (n * 4
+// bytes): the tile heads and their scan (n * 8 bytes) go back to the arena
+// before the mirrored cursors (n * 8 bytes) are taken, so the join's peak is
+// n * 24 bytes and the scans, below what is counted.
 constexpr uint64_t PAD = 256 * 64;  // alignment of up to 64 blocks
 
 uint64_t scan_state(uint64_t n) { return n / 8 + (1u << 20); }  // look-back scan state

@@ -1220,42 +1220,44 @@ __global__ __launch_bounds__(JB) void k_tile_ranges(JoinArgs a, uint32_t bound, 
     __shared__ uint32_t hist[QB];
     hist[threadIdx.x] = 0u;
     __syncthreads();
-    const uint64_t gid = (uint64_t)blockIdx.x * JB + threadIdx.x;
-    const uint32_t t = (uint32_t)(gid / LPT);
-    const int sub = (int)(gid % LPT);
-    const bool live = t < bound && t < *a.nTilesDev;
-    uint32_t pc = 0, cost = 0;
-    if (live) {
-        const int g = a.spanG > 0 ? a.spanG : 1;
-        const uint32_t cA = a.cellOf[a.tileStart[t]], cB = a.cellOf[a.tileStart[t + 1] - 1u];
-        uint32_t c[K];
+    const int sub = (int)(threadIdx.x % LPT);
+    const uint32_t nTiles = *a.nTilesDev;
+    constexpr uint32_t TPB = JB / LPT;  // tiles per block
+    for (uint64_t t = (uint64_t)blockIdx.x * TPB + threadIdx.x / LPT; t < bound; t += (uint64_t)gridDim.x * TPB) {
+        const bool live = t < nTiles;
+        uint32_t pc = 0, cost = 0;
+        if (live) {
+            const int g = a.spanG > 0 ? a.spanG : 1;
+            const uint32_t cA = a.cellOf[a.tileStart[t]], cB = a.cellOf[a.tileStart[t + 1] - 1u];
+            uint32_t c[K];
 #pragma unroll
-        for (int j = 0; j < K; j++) c[j] = a.cellCoord[(uint64_t)cA * K + j];
-        const TileSpan sp = tile_span<K>(a, g, c, a.cellLinear[cA], a.cellLinear[cB]);
-        int ng = 1;
+            for (int j = 0; j < K; j++) c[j] = a.cellCoord[(uint64_t)cA * K + j];
+            const TileSpan sp = tile_span<K>(a, g, c, a.cellLinear[cA], a.cellLinear[cB]);
+            int ng = 1;
 #pragma unroll
-        for (int j = 0; j < K; j++)
-            if (j >= g) ng *= 3;
-        for (int my = sub; my < ng; my += LPT) {
-            int od[K];
-            int64_t dl;
-            if (!span_group<K>(a, g, c, my, od, dl)) continue;
-            const uint32_t r = pos_lb(a, (uint64_t)((int64_t)sp.hi + dl)) - pos_lb(a, (uint64_t)((int64_t)sp.lo + dl));
-            pc += (r + cw - 1u) / cw;
-            cost += r;
+            for (int j = 0; j < K; j++)
+                if (j >= g) ng *= 3;
+            for (int my = sub; my < ng; my += LPT) {
+                int od[K];
+                int64_t dl;
+                if (!span_group<K>(a, g, c, my, od, dl)) continue;
+                const uint32_t r = pos_lb(a, (uint64_t)((int64_t)sp.hi + dl)) - pos_lb(a, (uint64_t)((int64_t)sp.lo + dl));
+                pc += (r + cw - 1u) / cw;
+                cost += r;
+            }
         }
-    }
 #pragma unroll
-    for (int off = LPT / 2; off > 0; off >>= 1) {
-        pc += __shfl_xor(pc, off, 64);
-        cost += __shfl_xor(cost, off, 64);
-    }
-    if (sub == 0) {
-        if (pieces && t < bound) pieces[t] = pc;
-        if (key && live) {
-            const uint32_t kk = cost_key(cost);
-            key[t] = kk;
-            atomicAdd(&hist[kk], 1u);
+        for (int off = LPT / 2; off > 0; off >>= 1) {
+            pc += __shfl_xor(pc, off, 64);
+            cost += __shfl_xor(cost, off, 64);
+        }
+        if (sub == 0) {
+            if (pieces) pieces[t] = pc;
+            if (key && live) {
+                const uint32_t kk = cost_key(cost);
+                key[t] = kk;
+                atomicAdd(&hist[kk], 1u);
+            }
         }
     }
     if (!bucket) return;
@@ -1408,31 +1410,31 @@ __global__ void k_sample_positions(const uint32_t *sortedIds, uint64_t n, uint64
 // 3,000 points of a 4-D grid (81 cells one after another).
 template <int K, int D>
 __global__ __launch_bounds__(JB) void k_sample_count(JoinArgs a, const uint32_t *list, uint64_t m) {
-    const uint64_t i = (uint64_t)blockIdx.x * WPB + (threadIdx.x >> 6);
-    if (i >= m) return;
     const int d = D > 0 ? D : a.d;
-    const uint32_t s = list[i], cell = a.cellOf[s];
-    uint32_t c[K];
+    for (uint64_t i = (uint64_t)blockIdx.x * WPB + (threadIdx.x >> 6); i < m; i += (uint64_t)gridDim.x * WPB) {
+        const uint32_t s = list[i], cell = a.cellOf[s];
+        uint32_t c[K];
 #pragma unroll
-    for (int j = 0; j < K; j++) c[j] = a.cellCoord[(uint64_t)cell * K + j];
-    const uint64_t linA = a.cellLinear[cell];
-    int noff = 1;
+        for (int j = 0; j < K; j++) c[j] = a.cellCoord[(uint64_t)cell * K + j];
+        const uint64_t linA = a.cellLinear[cell];
+        int noff = 1;
 #pragma unroll
-    for (int j = 0; j < K; j++) noff *= 3;
-    uint32_t hits = 0;
-    for (int my = (int)__lane_id(); my < noff; my += 64) {
-        int od[K];
-        int64_t dl;
-        if (!span_group<K>(a, 0, c, my, od, dl)) continue;
-        const int64_t b = find_cell(a, (uint64_t)((int64_t)linA + dl));
-        if (b < 0) continue;
-        const uint32_t t1 = a.cellStart[b + 1];
-        for (uint32_t t = a.cellStart[b]; t < t1; t++)
-            hits += d2_fp64<D>(a.pts + (uint64_t)s * d, a.pts + (uint64_t)t * d, d) <= a.T ? 1u : 0u;
+        for (int j = 0; j < K; j++) noff *= 3;
+        uint32_t hits = 0;
+        for (int my = (int)__lane_id(); my < noff; my += 64) {
+            int od[K];
+            int64_t dl;
+            if (!span_group<K>(a, 0, c, my, od, dl)) continue;
+            const int64_t b = find_cell(a, (uint64_t)((int64_t)linA + dl));
+            if (b < 0) continue;
+            const uint32_t t1 = a.cellStart[b + 1];
+            for (uint32_t t = a.cellStart[b]; t < t1; t++)
+                hits += d2_fp64<D>(a.pts + (uint64_t)s * d, a.pts + (uint64_t)t * d, d) <= a.T ? 1u : 0u;
+        }
+#pragma unroll
+        for (int off = 32; off > 0; off >>= 1) hits += __shfl_xor(hits, off, 64);
+        if (__lane_id() == 0) a.ownCnt[s] = hits;
     }
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) hits += __shfl_xor(hits, off, 64);
-    if (__lane_id() == 0) a.ownCnt[s] = hits;
 }
 
 __global__ void k_sum_gather(const uint32_t *v, const uint32_t *idx, uint64_t m, unsigned long long *out) {
@@ -1448,6 +1450,10 @@ static unsigned nblk(uint64_t n) {
     uint64_t g = (n + JB - 1) / JB;
     return (unsigned)(g ? g : 1);
 }
+// For kernels with many lanes per item, which go round: a launch may not
+// reach 2^32 threads, which 2^26 items of a wave each would.  2^20 blocks fill
+// the chip thousands of times, so sizes below that run as one round.
+static unsigned capped_blocks(uint64_t threads) { return std::min(nblk(threads), 1u << 20); }
 
 using JoinKernel = void (*)(JoinArgs);
 using SampleKernel = void (*)(JoinArgs, const uint32_t *, uint64_t);
@@ -1917,7 +1923,8 @@ sj_status launch_tile_ranges(const JoinArgs &a, int k, uint32_t bound, uint32_t 
         return SJ_ERR_UNSUPPORTED;
     }
     if (bound == 0) return SJ_OK;
-    hipLaunchKernelGGL(kfn, dim3(nblk((uint64_t)bound * lanes)), dim3(JB), 0, s, a, bound, cw, pieces, key, bucket);
+    hipLaunchKernelGGL(kfn, dim3(capped_blocks((uint64_t)bound * lanes)), dim3(JB), 0, s, a, bound, cw, pieces, key,
+                       bucket);
     SJ_LAUNCH_CHECK();
     return SJ_OK;
 }
@@ -2014,7 +2021,7 @@ static sj_status sample_count_list(sj_grid_s *g, const uint32_t *list, uint64_t 
     a.ownCnt = own.p;
     a.mirCnt = own.p;  // unused by FULL
     a.stat = stat.p;
-    hipLaunchKernelGGL(pick_sample(g->k, g->d), dim3(nblk(nsamp * 64)), dim3(JB), 0, s, a, list, nsamp);
+    hipLaunchKernelGGL(pick_sample(g->k, g->d), dim3(capped_blocks(nsamp * 64)), dim3(JB), 0, s, a, list, nsamp);
     SJ_LAUNCH_CHECK();
     hipLaunchKernelGGL(k_sum_gather, dim3(nblk(nsamp)), dim3(JB), 0, s, own.p, list, nsamp, stat.p + 5);
     SJ_LAUNCH_CHECK();

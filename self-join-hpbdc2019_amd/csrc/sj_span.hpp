@@ -383,11 +383,11 @@ __device__ __forceinline__ void span_flush(const JoinArgs &a, SpanLds &L, uint32
     const bool mirror = ok && a.form != SJ_FORM_FULL && !same && c >= a.wBegin && c < a.wEnd;
     if constexpr (PASS == PASS_COUNT) {
         const uint64_t slot = span_slots(a.mirCnt, mirror, c);
+        const uint32_t n = (uint32_t)__popcll(okm);
+        R.want += n;  // also past the end of the space: the whole demand
         if (rec.on) {
-            const uint32_t n = (uint32_t)__popcll(okm);
             uint64_t at, next;
             uint32_t room;
-            R.want += n;
             bool fits = !__ballot(slot > SPAN_SLOT_MAX);
             if (!fits && lane == 0) atomicAdd(&a.recCtr[REC_BAD], 1ull);
             fits = fits && span_rec_room(a, R, n, rec.n > 0, at, room, next);

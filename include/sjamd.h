@@ -101,9 +101,7 @@ typedef struct sj_stats {
     uint64_t num_batches;
     uint64_t candidates;         /* distance evaluations of the count pass */
     uint64_t fp32_band_pairs;    /* candidates re-decided in FP64 */
-    uint64_t fp32_misclassified; /* pairs whose plain FP32 decision was wrong
-                                  * (d = k >= 4: those the FP32 filter passed
-                                  * and FP64 rejected) */
+    uint64_t fp32_misclassified; /* pairs whose plain FP32 decision was wrong */
     uint64_t overflow_retries;
     double ms_grid;              /* device time, grid construction */
     double ms_workload;          /* device time, workload estimate + order */
@@ -322,7 +320,8 @@ SJ_API int32_t sj_mfma_band(double T, double R, int32_t d, float *alpha, float *
  * minus the tile's first point, rounded to the precision (FP64, or FP32 for
  * SJ_PREC_FP32_RECHECK), and all sums in that precision in any order, a pair
  * with d2_64 <= T has |q|^2 scale - 2 q.c <= t1 - |c|^2 scale; pairs that pass
- * are decided in FP64.  R bounds the differences of coordinates in a dim.
+ * are decided in FP64.  In FP32 a pair whose plain FP32 sum of squared
+ * differences is at most fl32(T) passes too (fp32_misclassified).  R bounds the differences of coordinates in a dim.
  * Returns 1 when the filter is used, 0 when its range does not hold T and R
  * (the join then evaluates the predicate for every candidate). */
 SJ_API int32_t sj_span_band(double T, double R, int32_t k, int32_t precision, double *scale, double *t1);

@@ -1704,6 +1704,10 @@ static int choose_span(const sj_grid_s *g) {
 // the canonical sum accepts true squared distances up to
 // T' = T / (1 - 1.01 (k + 3) 2^-53).  tiny covers denormals flushed in the
 // matrix cores.
+// FP32: pairs that a plain FP32 sum of squared differences accepts pass too
+// (sj_stats.fp32_misclassified counts the wrong ones among them).  That sum
+// errs by 2.02 k u s, the differences and the vectors' rounding by 8.01 u s;
+// 1.1 (3 KP + 8) u more in alpha covers the 2.02 KP + 8.01.
 // usable: squares of differences stay far from overflow, T far from underflow
 // (and from overflow: a grid's R is at least 2 eps, and the threshold must be
 // finite to reject the infinite norms of queries past the tile's end).
@@ -1712,7 +1716,7 @@ SpanBand span_band(double T, double R, int k, bool f32) {
     const int KP = (k + 3) / 4 * 4;
     SpanBand b;
     b.usable = f32 ? R < 1e15 && T > 1e-30 : R < 1e140 && T > 1e-280;
-    b.scale = 1.0 - 1.1 * (3 * KP + 16) * u;
+    b.scale = 1.0 - 1.1 * (f32 ? 6 * KP + 24 : 3 * KP + 16) * u;
     const double rho = 1.01 * (k + 3) * std::ldexp(1.0, -53), tiny = KP * std::ldexp(1.0, f32 ? -118 : -1000);
     b.T1 = T / (1.0 - rho) * (1.0 + 8.0 * u) + tiny;
     if (f32) {

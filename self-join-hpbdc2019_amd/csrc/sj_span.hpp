@@ -369,8 +369,17 @@ __device__ __forceinline__ void span_flush(const JoinArgs &a, SpanLds &L, uint32
     if (ok) {
         ok = d2_fp64<K>(xq, xc, K) <= a.T;
         if (F32 && PASS == PASS_COUNT && !a.spanDirect) {
+            // the plain FP32 decision: coordinates relative to the tile's
+            // first point, FMA chain in dimension order
+            float s32 = 0.0f;
+#pragma unroll
+            for (int j = 0; j < K; j++) {
+                const double ctr = a.pts[(uint64_t)ts0 * K + j];
+                const float f = (float)(xc[j] - ctr) - (float)(xq[j] - ctr);
+                s32 = j == 0 ? f * f : fmaf(f, f, s32);
+            }
             st.band++;
-            st.mis += ok ? 0u : 1u;
+            st.mis += ok != (s32 <= (float)a.T) ? 1u : 0u;
         }
     }
     const uint64_t okm = __ballot(ok);

@@ -84,6 +84,27 @@ def test_filter_passes_every_accepted_pair(d, eps, mult, prec):
             assert not ok.any()
 
 
+@pytest.mark.parametrize("d,eps,mult", CASES)
+def test_filter_passes_what_plain_fp32_accepts(d, eps, mult):
+    """pairs around the FP32 threshold whose FP32 sum of squared differences
+    accepts them, right or wrong (sj_stats.fp32_misclassified)"""
+    rng = np.random.default_rng(4000 + d)
+    T = O.eps_threshold(eps)
+    centre = rng.uniform(-mult * eps, mult * eps, size=d)
+    dirs = rng.normal(size=(200_000, d))
+    dirs /= np.linalg.norm(dirs, axis=1, keepdims=True)
+    p = rng.uniform(-mult * eps, mult * eps, size=dirs.shape)
+    q = p + dirs * (eps * (1.0 + rng.uniform(-1e-6, 8e-6 * mult, size=(len(dirs), 1))))
+    f = (q - centre).astype(np.float32) - (p - centre).astype(np.float32)
+    s32 = f[:, 0] * f[:, 0]
+    for j in range(1, d):
+        s32 = fma32(f[:, j], f[:, j], s32)
+    accepted = s32 <= np.float32(T)
+    assert (accepted & (O.dist2_batch(p, q) > T)).any()
+    for ok in _passes(p, q, centre, d, T, sjamd.FP32_RECHECK):
+        assert ok[accepted].all()
+
+
 @pytest.mark.parametrize("prec", [sjamd.FP64, sjamd.FP32_RECHECK])
 def test_filter_range(prec):
     """outside its range every pair goes to the predicate; inside it the

@@ -39,7 +39,7 @@
 // (no mirrored hit) << 63, in the order of the walk, so a row's own hits keep ascending positions.  A
 // tile's words start at recStart and fill the wave's blocks of REC_BLK words,
 // whose last word links to the next block; recN counts them.  The replaying
-// fill reads 64 words at a time and looks nothing up.
+// fill reads up to 256 words at a time and looks nothing up.
 // Bound: latency.  2M points uniform in 6-D, FP32+recheck: 9.4e9 pairs in
 // 3.6 ms, of which the matrix instructions are busy 1.05 ms and the vector
 // instructions 1.2 ms; 157 registers allow three waves per SIMD, and half of
@@ -66,6 +66,7 @@ constexpr uint64_t SPAN_SLOT_MAX = (1ull << 25) - 1;  // mirrored slots a record
 // the tile's query rows (all the replaying fill needs)
 struct SpanRows {
     uint64_t pos[64];       // fills: first entry of the query's row, NO_SLOT outside the window
+    uint32_t room[64];      // fills: own hits the row holds
     int32_t id[64];         // its point ID
     uint32_t own[64];       // its own hits so far
 };
@@ -413,7 +414,7 @@ __device__ __forceinline__ void span_flush(const JoinArgs &a, SpanLds &L, uint32
         const uint64_t p0 = L.pos[q];
         if (ok && p0 != NO_SLOT) {
             // more hits than the row has room for: count and fill disagree
-            if (rank < a.ownCnt[ts0 + q]) a.ids[p0 + rank] = (int32_t)a.origId[c];
+            if (rank < L.room[q]) a.ids[p0 + rank] = (int32_t)a.origId[c];
             else st.err++;
         }
         const uint64_t p = span_slots(a.mirCur, mirror, c);
@@ -433,6 +434,7 @@ __device__ __forceinline__ bool span_queries(const JoinArgs &a, SpanRows &L, uin
     L.own[lane] = 0u;
     if (PASS == PASS_FILL) {
         L.pos[lane] = ownW ? a.offS[s] - a.outBase : NO_SLOT;
+        L.room[lane] = ownW ? a.ownCnt[s] : 0u;
         L.id[lane] = (int32_t)a.origId[s];
     }
     return ownW;
@@ -567,12 +569,16 @@ __device__ __forceinline__ void process_span(const JoinArgs &a, uint32_t tile, S
         }
     } else {
         wave_lds_sync();
-        if (ownW && L.own[lane] != a.ownCnt[s]) st.err++;
+        if (ownW && L.own[lane] != L.room[lane]) st.err++;
     }
     wave_lds_sync();
 }
 
-// The same tile from the count pass's record.
+// The same tile from the count pass's record, up to 64 * REPLAY_U words at a
+// time: their loads, and then the loads that depend on them, are all in
+// flight together.  64 words at a time waited for two loads each: 2M points
+// in 4-D with 48 neighbours 832 -> 642 us, 20,000 with 1,000 670 -> 460 us.
+constexpr int REPLAY_U = 4;
 __device__ __forceinline__ void replay_span(const JoinArgs &a, uint32_t tile, SpanRows &L, LaneStats &st) {
     const unsigned lane = __lane_id();
     const uint32_t ts0 = uniform_u32(a.tileStart[tile]), ts1 = uniform_u32(a.tileStart[tile + 1]);
@@ -583,30 +589,50 @@ __device__ __forceinline__ void replay_span(const JoinArgs &a, uint32_t tile, Sp
     wave_lds_sync();
     while (left) {
         const uint32_t used = (uint32_t)(at % REC_BLK);
-        const uint32_t n = min(min(left, 64u), SPAN_LINK - used);
-        const bool live = lane < n;
-        const uint64_t w = live ? a.recMask[at + lane] : 0ull;
+        const uint32_t n = min(min(left, 64u * REPLAY_U), SPAN_LINK - used);
+        uint64_t w[REPLAY_U];
+#pragma unroll
+        for (int u = 0; u < REPLAY_U; u++) w[u] = lane + 64u * u < n ? a.recMask[at + lane + 64u * u] : 0ull;
         left -= n;
         at += n;
         if (left && at % REC_BLK == SPAN_LINK) at = uniform_u64(a.recMask[at]);
-        const uint32_t c = (uint32_t)w, q = (uint32_t)(w >> 32) & 63u;
-        const uint64_t peers = match6(__ballot(live), q);
-        const uint32_t rank = L.own[q] + popc_below64(peers);
-        wave_lds_sync();
-        if (live && popc_below64(peers) == 0) L.own[q] = rank + (uint32_t)__popcll(peers);
-        const uint64_t p0 = L.pos[q];
-        if (live && p0 != NO_SLOT) {
-            if (rank < a.ownCnt[ts0 + q]) a.ids[p0 + rank] = (int32_t)a.origId[c];
-            else st.err++;
+        int32_t id[REPLAY_U];
+        uint64_t p[REPLAY_U], lim[REPLAY_U];
+        bool mirror[REPLAY_U];
+#pragma unroll
+        for (int u = 0; u < REPLAY_U; u++) {
+            const bool live = lane + 64u * u < n;
+            const uint32_t c = (uint32_t)w[u];
+            id[u] = live ? (int32_t)a.origId[c] : 0;
+            mirror[u] = live && !(w[u] >> 63) && c >= a.wBegin && c < a.wEnd;
+            p[u] = lim[u] = 0;
+            if (mirror[u]) {
+                p[u] = a.offS[c] - a.outBase + a.ownCnt[c] + (w[u] >> 38);
+                lim[u] = a.offS[c + 1u] - a.outBase;
+            }
         }
-        if (live && !(w >> 63) && c >= a.wBegin && c < a.wEnd) {
-            const uint64_t p = a.offS[c] - a.outBase + a.ownCnt[c] + (w >> 38);
-            if (p < a.offS[c + 1u] - a.outBase) a.ids[p] = L.id[q];
-            else st.err++;
+#pragma unroll
+        for (int u = 0; u < REPLAY_U; u++) {
+            if (64u * u >= n) break;
+            const bool live = lane + 64u * u < n;
+            const uint32_t q = (uint32_t)(w[u] >> 32) & 63u;
+            const uint64_t peers = match6(__ballot(live), q);
+            const uint32_t rank = L.own[q] + popc_below64(peers);
+            wave_lds_sync();
+            if (live && popc_below64(peers) == 0) L.own[q] = rank + (uint32_t)__popcll(peers);
+            const uint64_t p0 = L.pos[q];
+            if (live && p0 != NO_SLOT) {
+                if (rank < L.room[q]) a.ids[p0 + rank] = id[u];
+                else st.err++;
+            }
+            if (mirror[u]) {
+                if (p[u] < lim[u]) a.ids[p[u]] = L.id[q];
+                else st.err++;
+            }
+            wave_lds_sync();
         }
-        wave_lds_sync();
     }
-    if (ownW && L.own[lane] != a.ownCnt[ts0 + lane]) st.err++;
+    if (ownW && L.own[lane] != L.room[lane]) st.err++;
     wave_lds_sync();
 }
 

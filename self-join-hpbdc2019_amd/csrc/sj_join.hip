@@ -810,43 +810,6 @@ __device__ __forceinline__ void process_tile(const JoinArgs &a, uint32_t tile, L
     st.err += err;
 }
 
-// The waves of a launch over the tiles of a: run(tile) for each, from the
-// work queue or in cell order, then the statistics and the record's demand.
-template <int PASS, class Run>
-__device__ __forceinline__ void tile_loop(const JoinArgs &a, LaneStats &st, TileRec &R, Run run) {
-    const unsigned wave = threadIdx.x >> 6;
-    const unsigned lane = __lane_id();
-    const uint32_t nTiles = *a.nTilesDev;
-    if (a.tileOrder) {
-        // work queue in QSLICES interleaved slices with one counter each:
-        // blocks are dealt to the XCDs round-robin, so a slice is served by
-        // the waves of one XCD.  A wave's first tile is static; the next
-        // grab is issued before the current tile runs, hiding its latency.
-        const uint32_t ns = min(gridDim.x, (uint32_t)QSLICES);
-        const uint32_t sl = blockIdx.x % ns;
-        const uint32_t nbl = (gridDim.x - sl + ns - 1) / ns;  // blocks of this slice
-        uint64_t i = (uint64_t)(blockIdx.x / ns) * WPB + wave;
-        for (;;) {
-            const uint64_t q = queue_entry(i, sl, ns);
-            if (q >= nTiles) break;
-            uint32_t nx = 0;
-            if (lane == 0) nx = atomicAdd(a.qctr + sl * QSTRIDE, 1u);
-            run(a.tileOrder[q]);
-            i = (uint64_t)nbl * WPB + readlane_u32(nx, 0);
-        }
-    } else {
-        // persistent grid-stride over the tiles in cell order
-        for (uint32_t tile = blockIdx.x * WPB + wave; tile < nTiles; tile += gridDim.x * WPB) run(tile);
-    }
-    flush_stats(a, st);
-    // mask words this wave's pieces needed, plus its last partial block,
-    // on the second word of the wave's counter slice
-    if (PASS == PASS_COUNT && a.recCtr && lane == 0) {
-        const uint32_t sl = (blockIdx.x * WPB + wave) % REC_NSLICE;
-        atomicAdd(&a.recCtr[REC_SLICE0 + sl * REC_STRIDE + 1], (unsigned long long)(R.want + REC_BLK));
-    }
-}
-
 template <int K, int D, int PASS, int PREC, bool RP, class LDS, bool DN = false>
 __device__ __forceinline__ void join_body(const JoinArgs &a, LDS *lds) {
     if (PASS == PASS_FILL && !fill_gate(a)) return;
@@ -876,30 +839,6 @@ template <int K, int D, int PASS, int PREC>
 __global__ __launch_bounds__(JB) void k_join(JoinArgs a) {
     __shared__ std::conditional_t<(D > 0 && K < SPAN_MINK), TileLds<D, PREC>, NoLds> lds[WPB];
     join_body<K, D, PASS, PREC, false>(a, lds);
-}
-
-// d = k >= 4: the span walk
-template <int K, int PASS, bool F32>
-__global__ __launch_bounds__(JB) __attribute__((amdgpu_waves_per_eu(F32 && K == 4 ? 4 : 3))) void k_span(JoinArgs a) {
-    __shared__ SpanLds lds[WPB];
-    if (PASS == PASS_FILL && !fill_gate(a)) return;
-    LaneStats st;
-    TileRec R;
-    tile_loop<PASS>(a, st, R, [&](uint32_t tile) __attribute__((always_inline)) {
-        process_span<K, PASS, F32>(a, tile, lds[threadIdx.x >> 6], st, R);
-    });
-}
-
-// and its fill from the record: no coordinates, one kernel for every k and
-// precision
-__global__ __launch_bounds__(JB) void k_span_rp(JoinArgs a) {
-    __shared__ SpanRows lds[WPB];
-    if (!fill_gate(a)) return;
-    LaneStats st;
-    TileRec R;
-    tile_loop<PASS_FILL>(a, st, R, [&](uint32_t tile) __attribute__((always_inline)) {
-        replay_span(a, tile, lds[threadIdx.x >> 6], st);
-    });
 }
 
 // k <= 2: four waves per SIMD (at most 128 VGPRs); measured faster at
@@ -969,7 +908,7 @@ __device__ __forceinline__ void many_tile(const JoinArgs &a, uint32_t tile, unsi
         if (PREC == 1 || a.d == K) {
             SpanLds &L = *reinterpret_cast<SpanLds *>(raw);
             if constexpr (RP) replay_span(a, tile, L, st);
-            else process_span<K, PASS, PREC == 1>(a, tile, L, st, R);
+            else process_span<K, PASS, PREC == 1, false>(a, tile, L, st, R);
         } else process_tile_wide<PASS>(a, tile, *reinterpret_cast<WideLds *>(raw), st, R);
     } else if constexpr (RP) {
         // the LDS tile walks replay their record; the wide walk keeps none
@@ -1455,7 +1394,6 @@ static unsigned nblk(uint64_t n) {
 // the chip thousands of times, so sizes below that run as one round.
 static unsigned capped_blocks(uint64_t threads) { return std::min(nblk(threads), 1u << 20); }
 
-using JoinKernel = void (*)(JoinArgs);
 using SampleKernel = void (*)(JoinArgs, const uint32_t *, uint64_t);
 
 template <int K, int D>
@@ -1536,24 +1474,6 @@ static TileRangesKernel pick_tile_ranges(int k, unsigned *lanes) {
     case 6: return k_tile_ranges<6, 64>;
     case 7: return k_tile_ranges<7, 64>;
     case 8: return k_tile_ranges<8, 64>;
-    }
-    return nullptr;
-}
-
-template <int K>
-static JoinKernel pick_span_k(int pass, int prec) {
-    if (pass == PASS_COUNT) return prec ? k_span<K, PASS_COUNT, true> : k_span<K, PASS_COUNT, false>;
-    return prec ? k_span<K, PASS_FILL, true> : k_span<K, PASS_FILL, false>;
-}
-
-static JoinKernel pick_span(int k, int pass, int prec, bool replay) {
-    if (replay) return k_span_rp;
-    switch (k) {
-    case 4: return pick_span_k<4>(pass, prec);
-    case 5: return pick_span_k<5>(pass, prec);
-    case 6: return pick_span_k<6>(pass, prec);
-    case 7: return pick_span_k<7>(pass, prec);
-    case 8: return pick_span_k<8>(pass, prec);
     }
     return nullptr;
 }
@@ -1739,6 +1659,13 @@ sj_status span_setup(sj_grid_s *g, JoinArgs &a, int prec) {
     for (int j = 0; j < g->k; j++) R = std::max(R, g->gp.maxArr[j] - g->gp.minArr[j]);
     const SpanBand b = span_band(a.T, R, g->k, prec == SJ_PREC_FP32_RECHECK);
     a.spanDirect = !b.usable;
+    // From 64 points per occupied cell a block of 16 candidates lies in one or
+    // two cells, and whole blocks may be hits.  4,000 points in one cell, 4-D /
+    // 8-D: 5.9 / 6.2 ms without these kernels, 1.6 / 1.9 ms with them; 20,000
+    // uniform points with 1,000 neighbours, where few blocks are dense: 1.87 /
+    // 1.91 ms without, 1.79 / 2.00 ms with.  Below the line blocks are sparse,
+    // and the larger kernels cost 3 to 5% (6-D and 8-D at 32 and 24 neighbours).
+    a.spanDense = g->n >= 64 * g->nNonEmpty;
     a.spanScale = b.scale;
     a.spanT1 = b.T1;
     SJ_TRY(g->posPk.alloc(&g->ctx->pool, g->n));
@@ -1881,7 +1808,7 @@ static sj_status launch_join(sj_grid_s *g, const JoinArgs &a, int pass, int prec
         return launch_join_mfma(ar, pass, g->ctx->cu_count, s, true);
     }
     JoinKernel kfn;
-    if (a.spanG > 0) kfn = pick_span(g->k, pass, prec, replay);
+    if (a.spanG > 0) kfn = pick_span(g->k, pass, prec, replay, a.spanDense != 0);
     else if (a.posLB && g->k == g->d && g->k == 2) kfn = pick_dense2(pass, prec, replay);
     else kfn = replay ? pick_replay(g->k, prec) : pick_kernel(g->k, g->d, pass, prec);
     if (!kfn) {

@@ -1,0 +1,52 @@
+// Kernels of the span walk (d = k = 4..8); the device side is sj_span.hpp.
+#include "sj_span.hpp"
+
+namespace sj {
+
+template <int K, int PASS, bool F32, bool DENSE>
+__global__ __launch_bounds__(JB) __attribute__((amdgpu_waves_per_eu(F32 && K == 4 ? 4 : 3))) void k_span(JoinArgs a) {
+    __shared__ SpanLds lds[WPB];
+    if (PASS == PASS_FILL && !fill_gate(a)) return;
+    LaneStats st;
+    TileRec R;
+    tile_loop<PASS>(a, st, R, [&](uint32_t tile) __attribute__((always_inline)) {
+        process_span<K, PASS, F32, DENSE>(a, tile, lds[threadIdx.x >> 6], st, R);
+    });
+}
+
+// The fill from the record: no coordinates, one kernel for every k and
+// precision
+__global__ __launch_bounds__(JB) void k_span_rp(JoinArgs a) {
+    __shared__ SpanRows lds[WPB];
+    if (!fill_gate(a)) return;
+    LaneStats st;
+    TileRec R;
+    tile_loop<PASS_FILL>(a, st, R, [&](uint32_t tile) __attribute__((always_inline)) {
+        replay_span(a, tile, lds[threadIdx.x >> 6], st);
+    });
+}
+
+template <int K, bool DENSE>
+static JoinKernel pick_k(int pass, int prec) {
+    if (pass == PASS_COUNT) return prec ? k_span<K, PASS_COUNT, true, DENSE> : k_span<K, PASS_COUNT, false, DENSE>;
+    return prec ? k_span<K, PASS_FILL, true, DENSE> : k_span<K, PASS_FILL, false, DENSE>;
+}
+
+template <bool DENSE>
+static JoinKernel pick(int k, int pass, int prec) {
+    switch (k) {
+    case 4: return pick_k<4, DENSE>(pass, prec);
+    case 5: return pick_k<5, DENSE>(pass, prec);
+    case 6: return pick_k<6, DENSE>(pass, prec);
+    case 7: return pick_k<7, DENSE>(pass, prec);
+    case 8: return pick_k<8, DENSE>(pass, prec);
+    }
+    return nullptr;
+}
+
+JoinKernel pick_span(int k, int pass, int prec, bool replay, bool dense) {
+    if (replay) return k_span_rp;
+    return dense ? pick<true>(k, pass, prec) : pick<false>(k, pass, prec);
+}
+
+}  // namespace sj

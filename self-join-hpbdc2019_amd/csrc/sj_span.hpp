@@ -36,10 +36,11 @@
 // so there the coordinates themselves are compared.
 //
 // Hit record: one word per hit, candidate | query << 32 | mirrored slot << 38 |
-// (no mirrored hit) << 63, in the order of the walk, so a row's own hits keep ascending positions.  A
-// tile's words start at recStart and fill the wave's blocks of REC_BLK words,
-// whose last word links to the next block; recN counts them.  The replaying
-// fill reads up to 256 words at a time and looks nothing up.
+// (no mirrored hit) << 63, in the order of the walk, so a row's own hits keep
+// ascending positions; blocks of candidates decided whole (span_dense) as masks
+// of queries.  A tile's words start at recStart and fill the wave's blocks of
+// REC_BLK words, whose last word links to the next block; recN counts them.
+// The replaying fill reads up to 256 words at a time and looks nothing up.
 // Bound: latency.  2M points uniform in 6-D, FP32+recheck: 9.4e9 pairs in
 // 3.6 ms, of which the matrix instructions are busy 1.05 ms and the vector
 // instructions 1.2 ms; 157 registers allow three waves per SIMD, and half of
@@ -62,6 +63,11 @@ constexpr int SPAN_MINK = 4;
 constexpr uint32_t SPAN_BUF = 63 + 64 * 16;        // gathered pairs: 64 x 16 come in on top of at most 63
 constexpr uint32_t SPAN_LINK = REC_BLK - 1u;       // a block's link to the next
 constexpr uint64_t SPAN_SLOT_MAX = (1ull << 25) - 1;  // mirrored slots a record word holds
+// Other record words, told by two of the bits that a word without a mirrored
+// hit leaves 0: the head of a block of candidates (first | number << 32, then
+// three words each: queries with hits, with mirrored hits, first slot), and
+// the rest of the record block unused.
+constexpr uint64_t SPAN_BLOCK = 3ull << 62, SPAN_SKIP = 5ull << 61;
 
 // the tile's query rows (all the replaying fill needs)
 struct SpanRows {
@@ -331,6 +337,64 @@ __device__ __forceinline__ uint64_t span_slots(Ctr *ctr, bool mirror, uint32_t c
     return own ? base : ((((uint64_t)hi << 32) | lo) + popc_below64(group));
 }
 
+// Whether a query (cells pkq, own cell from position cs0) claims candidate c
+// (same: in its own cell), z = pk_diff of their cells.
+template <int K>
+__device__ __forceinline__ bool span_claim(const JoinArgs &a, uint32_t z, uint32_t pkq, uint32_t c, uint32_t cs0,
+                                           bool same) {
+    if (pk_far(z)) return false;
+    if (a.form == SJ_FORM_LID) return c >= cs0;
+    if (a.form == SJ_FORM_FULL || same) return true;
+    uint32_t cp[K];  // claims reads only the parities
+    int o[K];
+#pragma unroll
+    for (int j = 0; j < K; j++) {
+        const uint32_t f = (z >> (4 * j)) & 3u;
+        o[j] = f == 3u ? -1 : (int)f;
+        cp[j] = (pkq >> (4 * j)) & 3u;
+    }
+    return claims<K>(a.form, cp, o, 0, 0);
+}
+
+// Records the hits of the lanes in okm: candidate c, query q, mirrored hits'
+// slots.
+__device__ __forceinline__ void span_record(const JoinArgs &a, TileRec &R, SpanRec &rec, uint64_t okm, bool ok,
+                                            uint32_t c, uint32_t q, bool mirror, uint64_t slot) {
+    const uint32_t n = (uint32_t)__popcll(okm);
+    R.want += n;  // also past the end of the space: the whole demand
+    if (!rec.on) return;
+    uint64_t at, next;
+    uint32_t room;
+    slot = mirror ? slot : 0ull;
+    bool fits = !__ballot(slot > SPAN_SLOT_MAX);
+    if (!fits && __lane_id() == 0) atomicAdd(&a.recCtr[REC_BAD], 1ull);
+    fits = fits && span_rec_room(a, R, n, rec.n > 0, at, room, next);
+    rec.on = fits;
+    if (!fits) return;
+    if (rec.n == 0) rec.start = at;
+    if (rec.n == 0 && at == next) room = n;  // all of them in the new block
+    const uint32_t i = popc_below64(okm);
+    if (ok)
+        a.recMask[i < room ? at + i : next + (i - room)] =
+            (uint64_t)c | ((uint64_t)q << 32) | (slot << 38) | (mirror ? 0ull : 1ull << 63);
+    rec.n += n;
+}
+
+// The plain FP32 decision of a pair: coordinates relative to the tile's first
+// point, FMA chain in dimension order.
+template <int K>
+__device__ __forceinline__ bool span_plain32(const JoinArgs &a, uint32_t ts0, const double (&xq)[K],
+                                             const double (&xc)[K]) {
+    float s32 = 0.0f;
+#pragma unroll
+    for (int j = 0; j < K; j++) {
+        const double ctr = a.pts[(uint64_t)ts0 * K + j];
+        const float f = (float)(xc[j] - ctr) - (float)(xq[j] - ctr);
+        s32 = j == 0 ? f * f : fmaf(f, f, s32);
+    }
+    return s32 <= (float)a.T;
+}
+
 // Decides the nh <= 64 gathered pairs from buffer position head, one per
 // lane, and counts and records them, or writes them to their rows.
 template <int K, int PASS, bool F32>
@@ -347,40 +411,18 @@ __device__ __forceinline__ void span_flush(const JoinArgs &a, SpanLds &L, uint32
     for (int j = 0; j < K; j++) xq[j] = a.pts[(uint64_t)(ts0 + q) * K + j];
     const uint32_t z = pk_diff(a.posPk[c], pkA);
     const bool same = c >= cs0 && c < cs1;  // the query's own cell
-    bool ok = lane < nh && !pk_far(z);
+    bool ok = lane < nh && span_claim<K>(a, z, pkA, c, cs0, same);
     if (a.spanDirect) {
         const uint32_t *cc = a.cellCoord + (uint64_t)a.cellOf[c] * K;
         const uint32_t *cq = a.cellCoord + (uint64_t)a.cellOf[ts0 + q] * K;
 #pragma unroll
         for (int j = 0; j < K; j++) ok = ok && cc[j] - cq[j] + 1u <= 2u;
     }
-    if (a.form == SJ_FORM_LID) {
-        ok = ok && c >= cs0;
-    } else if (a.form != SJ_FORM_FULL) {
-        uint32_t cp[K];  // claims reads only the parities
-        int o[K];
-#pragma unroll
-        for (int j = 0; j < K; j++) {
-            const uint32_t f = (z >> (4 * j)) & 3u;
-            o[j] = f == 3u ? -1 : (int)f;
-            cp[j] = (pkA >> (4 * j)) & 3u;
-        }
-        ok = ok && (same || claims<K>(a.form, cp, o, 0, 0));
-    }
     if (ok) {
         ok = d2_fp64<K>(xq, xc, K) <= a.T;
         if (F32 && PASS == PASS_COUNT && !a.spanDirect) {
-            // the plain FP32 decision: coordinates relative to the tile's
-            // first point, FMA chain in dimension order
-            float s32 = 0.0f;
-#pragma unroll
-            for (int j = 0; j < K; j++) {
-                const double ctr = a.pts[(uint64_t)ts0 * K + j];
-                const float f = (float)(xc[j] - ctr) - (float)(xq[j] - ctr);
-                s32 = j == 0 ? f * f : fmaf(f, f, s32);
-            }
             st.band++;
-            st.mis += ok != (s32 <= (float)a.T) ? 1u : 0u;
+            st.mis += ok != span_plain32<K>(a, ts0, xq, xc) ? 1u : 0u;
         }
     }
     const uint64_t okm = __ballot(ok);
@@ -393,23 +435,7 @@ __device__ __forceinline__ void span_flush(const JoinArgs &a, SpanLds &L, uint32
     const bool mirror = ok && a.form != SJ_FORM_FULL && !same && c >= a.wBegin && c < a.wEnd;
     if constexpr (PASS == PASS_COUNT) {
         const uint64_t slot = span_slots(a.mirCnt, mirror, c);
-        const uint32_t n = (uint32_t)__popcll(okm);
-        R.want += n;  // also past the end of the space: the whole demand
-        if (rec.on) {
-            uint64_t at, next;
-            uint32_t room;
-            bool fits = !__ballot(slot > SPAN_SLOT_MAX);
-            if (!fits && lane == 0) atomicAdd(&a.recCtr[REC_BAD], 1ull);
-            fits = fits && span_rec_room(a, R, n, rec.n > 0, at, room, next);
-            rec.on = fits;
-            if (fits) {
-                if (rec.n == 0) rec.start = at;
-                if (rec.n == 0 && at == next) room = n;  // all of them in the new block
-                const uint32_t i = popc_below64(okm);
-                if (ok) a.recMask[i < room ? at + i : next + (i - room)] = (uint64_t)c | ((uint64_t)q << 32) | (slot << 38) | (mirror ? 0ull : 1ull << 63);
-                rec.n += n;
-            }
-        }
+        span_record(a, R, rec, okm, ok, c, q, mirror, slot);
     } else {
         const uint64_t p0 = L.pos[q];
         if (ok && p0 != NO_SLOT) {
@@ -423,6 +449,152 @@ __device__ __forceinline__ void span_flush(const JoinArgs &a, SpanLds &L, uint32
             else st.err++;
         }
     }
+}
+
+__device__ __forceinline__ double readlane_f64(double v, uint32_t l) {
+    return __longlong_as_double((long long)readlane_u64((uint64_t)__double_as_longlong(v), (int)l));
+}
+
+// Room for a run of n < 64 record words in one block: what is left of a
+// block too short for it is skipped (SPAN_SKIP).  False when the record space
+// is exhausted.
+__device__ __forceinline__ bool span_rec_run(const JoinArgs &a, TileRec &R, SpanRec &rec, uint32_t n, uint64_t &at) {
+    uint64_t next;
+    uint32_t room;
+    const uint32_t left = R.used < SPAN_LINK ? SPAN_LINK - R.used : 0u;
+    if (R.ok && left > 0 && left < n) {
+        if (rec.n) {
+            if (__lane_id() == 0) a.recMask[R.blk + R.used] = SPAN_SKIP;
+            rec.n++;
+        }
+        R.used = SPAN_LINK;
+    }
+    rec.on = span_rec_room(a, R, n, rec.n > 0, at, room, next);
+    if (!rec.on) return false;
+    if (room < n) at = next;
+    if (rec.n == 0) rec.start = at;
+    rec.n += n;
+    return true;
+}
+
+// Writes the hits of nc <= 16 candidates to their rows, lane q those of query
+// q.  Lane i holds candidate i's values: the queries with hits and with
+// mirrored hits, its ID, the row position of its first mirrored hit and its
+// row's end.
+__device__ __forceinline__ void span_emit(const JoinArgs &a, SpanRows &L, uint32_t nc, uint64_t okl, uint64_t mml,
+                                          int32_t idl, uint64_t base, uint64_t lim, LaneStats &st) {
+    const unsigned lane = __lane_id();
+    const uint64_t p0 = L.pos[lane];
+    const uint32_t room = L.room[lane];
+    const int32_t idq = L.id[lane];
+    uint32_t own = L.own[lane];
+#pragma unroll 1
+    for (uint32_t i = 0; i < nc; i++) {
+        const uint64_t okm = readlane_u64(okl, (int)i), mm = readlane_u64(mml, (int)i);
+        const int32_t id = (int32_t)readlane_u32((uint32_t)idl, (int)i);
+        if ((okm >> lane) & 1ull) {
+            if (p0 != NO_SLOT) {
+                // more hits than the row has room for: count and fill disagree
+                if (own < room) a.ids[p0 + own] = id;
+                else st.err++;
+            }
+            own++;
+        }
+        if (mm) {
+            const uint64_t p = readlane_u64(base, (int)i) + popc_below64(mm), end = readlane_u64(lim, (int)i);
+            if ((mm >> lane) & 1ull) {
+                if (p < end) a.ids[p] = idq;
+                else st.err++;
+            }
+        }
+    }
+    L.own[lane] = own;
+}
+
+// The 16 candidates [t0, ..) below t1, many of whose pairs are hits: lane q
+// decides all of them for query q, the candidates' coordinates broadcast from
+// the lanes that hold them (x, as SpanQuery::fetch leaves them).  One round
+// of loads and atomics and one run of record words serve up to 1,024 pairs,
+// where span_flush has one per 64.  Returns the hits.
+constexpr uint32_t SPAN_DENSE = 256;  // pairs of 1,024: four rounds of span_flush or one of span_dense
+template <int K, int PASS, bool F32>
+__device__ __forceinline__ uint32_t span_dense(const JoinArgs &a, SpanLds &L, uint32_t ts0, uint32_t m, uint32_t t0,
+                                               uint32_t t1, const double (&x)[(K + 3) / 4], LaneStats &st, TileRec &R,
+                                               SpanRec &rec) {
+    const unsigned lane = __lane_id();
+    double xq[K];
+#pragma unroll
+    for (int j = 0; j < K; j++) xq[j] = a.pts[(uint64_t)(ts0 + min(lane, m - 1u)) * K + j];
+    const uint32_t cp = min(t0 + (lane & 15u), t1 - 1u), nc = min(16u, t1 - t0);
+    // the candidates that the query claims, and those that get a mirrored hit
+    uint32_t may = (1u << nc) - 1u, mirrored = 0u;
+    {
+        const uint32_t pkq = L.pk[lane], cs0 = L.cs0[lane], cs1 = L.cs1[lane];
+        // nothing to find out when the block lies in every query's own cell
+        if (__ballot(lane < m && (t0 < cs0 || t0 + nc > cs1))) {
+            const uint32_t pkl = a.posPk[cp];
+            may = 0u;
+#pragma unroll 1
+            for (uint32_t i = 0; i < nc; i++) {
+                const uint32_t c = t0 + i;
+                const bool same = c >= cs0 && c < cs1;
+                const bool ok = span_claim<K>(a, pk_diff(readlane_u32(pkl, (int)i), pkq), pkq, c, cs0, same);
+                may |= ok ? 1u << i : 0u;
+                mirrored |= ok && !same ? 1u << i : 0u;
+            }
+            if (a.form == SJ_FORM_FULL) mirrored = 0u;
+            mirrored &= (uint32_t)range_bits(t0, a.wBegin, a.wEnd);
+        }
+        may = lane < m ? may : 0u;
+    }
+    uint32_t near = 0u, plain = 0u;
+#pragma unroll 4
+    for (uint32_t i = 0; i < 16u; i++) {
+        double xc[K];
+#pragma unroll
+        for (int j = 0; j < K; j++) xc[j] = readlane_f64(x[j / 4], i + 16u * (j % 4));
+        near |= d2_fp64<K>(xq, xc, K) <= a.T ? 1u << i : 0u;
+        if (F32 && PASS == PASS_COUNT) plain |= span_plain32<K>(a, ts0, xq, xc) ? 1u << i : 0u;
+    }
+    if (F32 && PASS == PASS_COUNT) {
+        st.band += (uint32_t)__popc(may);
+        st.mis += (uint32_t)__popc((near ^ plain) & may);
+    }
+    const uint32_t hit = near & may, mir = hit & mirrored;
+    uint32_t total = 0;
+    uint64_t okl = 0, mml = 0;  // lane i: the queries with a (mirrored) hit on candidate t0 + i
+    for (uint32_t i = 0; i < nc; i++) {
+        const uint64_t okm = __ballot((hit >> i) & 1u), mm = __ballot((mir >> i) & 1u);
+        okl = lane == i ? okm : okl;
+        mml = lane == i ? mm : mml;
+        total += (uint32_t)__popcll(okm);
+    }
+    // a slot per mirrored hit
+    uint64_t base = 0;
+    const uint32_t cnt = (uint32_t)__popcll(mml);
+    if (cnt) {
+        if constexpr (PASS == PASS_COUNT) base = atomicAdd(&a.mirCnt[cp], cnt);
+        else base = atomicAdd(&a.mirCur[cp], (unsigned long long)cnt);
+    }
+    if constexpr (PASS == PASS_COUNT) {
+        L.own[lane] += (uint32_t)__popc(hit);
+        R.want += 1u + 3u * nc;
+        uint64_t at;
+        if (rec.on && span_rec_run(a, R, rec, 1u + 3u * nc, at)) {
+            if (lane == 0) a.recMask[at] = SPAN_BLOCK | ((uint64_t)nc << 32) | t0;
+            if (lane < nc) {
+                uint64_t *e = a.recMask + at + 1u + 3u * lane;
+                e[0] = okl;
+                e[1] = mml;
+                e[2] = base;
+            }
+        }
+    } else {
+        const bool inW = lane < nc && cp >= a.wBegin && cp < a.wEnd;
+        span_emit(a, L, nc, okl, mml, (int32_t)a.origId[cp], base, inW ? a.offS[cp + 1u] - a.outBase : 0ull, st);
+    }
+    wave_lds_sync();
+    return total;
 }
 
 // The tile's queries into LDS (lane q holds query q).
@@ -440,8 +612,10 @@ __device__ __forceinline__ bool span_queries(const JoinArgs &a, SpanRows &L, uin
     return ownW;
 }
 
-// One tile of the span walk.
-template <int K, int PASS, bool F32>
+// One tile of the span walk.  DENSE: blocks in which many pairs pass the filter
+// are decided whole (span_dense), without the filter while they follow one
+// another.
+template <int K, int PASS, bool F32, bool DENSE>
 __device__ __forceinline__ void process_span(const JoinArgs &a, uint32_t tile, SpanLds &L, LaneStats &st,
                                              TileRec &R) {
     const unsigned lane = __lane_id();
@@ -505,6 +679,7 @@ __device__ __forceinline__ void process_span(const JoinArgs &a, uint32_t tile, S
     };
     using T = typename SpanMma<F32>::T;
     const T scale = (T)a.spanScale, T1 = (T)a.spanT1;
+    bool rich = false;  // the last block was dense
 
     int ng = 1;
 #pragma unroll
@@ -552,8 +727,21 @@ __device__ __forceinline__ void process_span(const JoinArgs &a, uint32_t tile, S
             for (uint32_t t0 = u0; t0 < u1; t0 += 16u) {
                 // the next candidates' coordinates are on their way meanwhile
                 Q.fetch(a, min(t0 + 16u + (lane & 15u), u1 - 1u), nx);
-                Q.filter(t0, u1, x, scale, T1, gather);
-                if (nh >= 64u) drain(false);
+                bool dense = DENSE && rich;
+                if (!dense) {
+                    const uint32_t before = nh;
+                    Q.filter(t0, u1, x, scale, T1, gather);
+                    if (DENSE && nh - before >= SPAN_DENSE) {
+                        // decided whole, after the pairs gathered before
+                        nh = before;
+                        dense = true;
+                    }
+                    if (dense ? nh > 0u : nh >= 64u) drain(dense);
+                }
+                if constexpr (DENSE) {
+                    if (dense)
+                        rich = span_dense<K, PASS, F32>(a, L, ts0, m, t0, u1, x, st, R, rec) >= SPAN_DENSE;
+                }
 #pragma unroll
                 for (int h = 0; h < Q.H; h++) x[h] = nx[h];
             }
@@ -575,9 +763,9 @@ __device__ __forceinline__ void process_span(const JoinArgs &a, uint32_t tile, S
 }
 
 // The same tile from the count pass's record, up to 64 * REPLAY_U words at a
-// time: their loads, and then the loads that depend on them, are all in
-// flight together.  64 words at a time waited for two loads each: 2M points
-// in 4-D with 48 neighbours 832 -> 642 us, 20,000 with 1,000 670 -> 460 us.
+// time: the loads that depend on them are all in flight together, as are the
+// next words.  64 words at a time waited for two loads each: 2M points in
+// 4-D with 48 neighbours 832 -> 657 us, 20,000 with 1,000 670 -> 473 us.
 constexpr int REPLAY_U = 4;
 __device__ __forceinline__ void replay_span(const JoinArgs &a, uint32_t tile, SpanRows &L, LaneStats &st) {
     const unsigned lane = __lane_id();
@@ -586,16 +774,61 @@ __device__ __forceinline__ void replay_span(const JoinArgs &a, uint32_t tile, Sp
     const bool ownW = span_queries<PASS_FILL>(a, L, ts0, ts1);
     uint32_t left = uniform_u32(a.recN[tile]);
     uint64_t at = uniform_u64(a.recStart[tile]);
+    // the words from `at` on, within the tile's and the record block's
+    uint64_t next[REPLAY_U];
+    uint32_t nNext;
+    auto load = [&]() __attribute__((always_inline)) {
+        nNext = min(min(left, 64u * REPLAY_U), SPAN_LINK - (uint32_t)(at % REC_BLK));
+#pragma unroll
+        for (int u = 0; u < REPLAY_U; u++)
+            next[u] = lane + 64u * u < nNext ? a.recMask[at + lane + 64u * u] : 0ull;
+    };
+    if (left) load();
     wave_lds_sync();
     while (left) {
-        const uint32_t used = (uint32_t)(at % REC_BLK);
-        const uint32_t n = min(min(left, 64u * REPLAY_U), SPAN_LINK - used);
         uint64_t w[REPLAY_U];
 #pragma unroll
-        for (int u = 0; u < REPLAY_U; u++) w[u] = lane + 64u * u < n ? a.recMask[at + lane + 64u * u] : 0ull;
+        for (int u = 0; u < REPLAY_U; u++) w[u] = next[u];
+        uint32_t n = nNext;
+        // up to the first word that is not a hit
+        uint64_t special = 0;
+#pragma unroll
+        for (int u = REPLAY_U - 1; u >= 0; u--) {
+            const uint64_t b = __ballot((w[u] >> 61) > 4ull);
+            if (b) {
+                n = 64u * u + (uint32_t)__builtin_ctzll(b);
+                special = readlane_u64(w[u], __builtin_ctzll(b));
+            }
+        }
+        const bool block = special >= SPAN_BLOCK;
+        const uint32_t nc = block ? (uint32_t)(special >> 32) & 31u : 0u;
         left -= n;
         at += n;
-        if (left && at % REC_BLK == SPAN_LINK) at = uniform_u64(a.recMask[at]);
+        // a block's words: lane i those of its candidate i
+        uint64_t okl = 0, mml = 0, base = 0, end = 0;
+        int32_t idl = 0;
+        if (lane < nc) {
+            const uint32_t c = (uint32_t)special + lane;
+            const uint64_t *e = a.recMask + at + 1u + 3u * lane;
+            okl = e[0];
+            idl = (int32_t)a.origId[c];
+            if (c >= a.wBegin && c < a.wEnd) {
+                mml = e[1];
+                base = a.offS[c] - a.outBase + a.ownCnt[c] + e[2];
+                end = a.offS[c + 1u] - a.outBase;
+            }
+        }
+        if (block) {
+            left -= 1u + 3u * nc;
+            at += 1u + 3u * nc;
+        } else if (special) {
+            left--;
+            at = at / REC_BLK * REC_BLK + SPAN_LINK;
+        }
+        if (left) {
+            if (at % REC_BLK == SPAN_LINK) at = uniform_u64(a.recMask[at]);
+            load();
+        }
         int32_t id[REPLAY_U];
         uint64_t p[REPLAY_U], lim[REPLAY_U];
         bool mirror[REPLAY_U];
@@ -629,6 +862,10 @@ __device__ __forceinline__ void replay_span(const JoinArgs &a, uint32_t tile, Sp
                 if (p[u] < lim[u]) a.ids[p[u]] = L.id[q];
                 else st.err++;
             }
+            wave_lds_sync();
+        }
+        if (nc) {
+            span_emit(a, L, nc, okl, mml, idl, base, end, st);
             wave_lds_sync();
         }
     }

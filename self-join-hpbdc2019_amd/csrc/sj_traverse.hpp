@@ -74,6 +74,7 @@ struct JoinArgs {
     int spanG;
     uint32_t nPts;             // points in the sorted arrays
     int spanDirect;            // no filter: the predicate for every candidate
+    int spanDense;             // kernels that decide blocks with many hits whole
     double spanScale, spanT1;  // filter: norms scaled by 1 - alpha, threshold
     const uint32_t *posPk;     // per point: cell coordinates modulo 4, 4 bits per dim
     uint32_t *recN;            // record words per tile
@@ -217,6 +218,43 @@ __device__ __forceinline__ void flush_stats(const JoinArgs &a, const LaneStats &
         if (m) atomicAdd(&a.stat[STAT_MIS], (unsigned long long)m);
         if (e) atomicAdd(&a.stat[STAT_ERR], (unsigned long long)e);
         if (f) atomicAdd(&a.stat[STAT_FALLBACK], (unsigned long long)f);
+    }
+}
+
+// The waves of a launch over the tiles of a: run(tile) for each, from the
+// work queue or in cell order, then the statistics and the record's demand.
+template <int PASS, class Run>
+__device__ __forceinline__ void tile_loop(const JoinArgs &a, LaneStats &st, TileRec &R, Run run) {
+    const unsigned wave = threadIdx.x >> 6;
+    const unsigned lane = __lane_id();
+    const uint32_t nTiles = *a.nTilesDev;
+    if (a.tileOrder) {
+        // work queue in QSLICES interleaved slices with one counter each:
+        // blocks are dealt to the XCDs round-robin, so a slice is served by
+        // the waves of one XCD.  A wave's first tile is static; the next
+        // grab is issued before the current tile runs, hiding its latency.
+        const uint32_t ns = min(gridDim.x, (uint32_t)QSLICES);
+        const uint32_t sl = blockIdx.x % ns;
+        const uint32_t nbl = (gridDim.x - sl + ns - 1) / ns;  // blocks of this slice
+        uint64_t i = (uint64_t)(blockIdx.x / ns) * WPB + wave;
+        for (;;) {
+            const uint64_t q = queue_entry(i, sl, ns);
+            if (q >= nTiles) break;
+            uint32_t nx = 0;
+            if (lane == 0) nx = atomicAdd(a.qctr + sl * QSTRIDE, 1u);
+            run(a.tileOrder[q]);
+            i = (uint64_t)nbl * WPB + readlane_u32(nx, 0);
+        }
+    } else {
+        // persistent grid-stride over the tiles in cell order
+        for (uint32_t tile = blockIdx.x * WPB + wave; tile < nTiles; tile += gridDim.x * WPB) run(tile);
+    }
+    flush_stats(a, st);
+    // mask words this wave's pieces needed, plus its last partial block,
+    // on the second word of the wave's counter slice
+    if (PASS == PASS_COUNT && a.recCtr && lane == 0) {
+        const uint32_t sl = (blockIdx.x * WPB + wave) % REC_NSLICE;
+        atomicAdd(&a.recCtr[REC_SLICE0 + sl * REC_STRIDE + 1], (unsigned long long)(R.want + REC_BLK));
     }
 }
 
@@ -589,6 +627,9 @@ struct SpanBand {
     bool usable;
 };
 SpanBand span_band(double T, double R, int k, bool f32);
+using JoinKernel = void (*)(JoinArgs);
+// Kernel of the span walk (sj_span.hip): count, evaluating or replaying fill.
+JoinKernel pick_span(int k, int pass, int prec, bool replay, bool dense);
 // Chooses the span walk for joins with d = k >= 4 and sets its fields.
 sj_status span_setup(sj_grid_s *g, JoinArgs &a, int prec);
 

@@ -907,8 +907,8 @@ __device__ __forceinline__ void many_tile(const JoinArgs &a, uint32_t tile, unsi
         // the wide walk (FP64 only) keeps no record
         if (PREC == 1 || a.d == K) {
             SpanLds &L = *reinterpret_cast<SpanLds *>(raw);
-            if constexpr (RP) replay_span(a, tile, L, st);
-            else process_span<K, PASS, PREC == 1, false>(a, tile, L, st, R);
+            if constexpr (RP) replay_span_many(a, tile, L, st);
+            else process_span<K, PASS, PREC == 1, SPAN_ANY>(a, tile, L, st, R);
         } else process_tile_wide<PASS>(a, tile, *reinterpret_cast<WideLds *>(raw), st, R);
     } else if constexpr (RP) {
         // the LDS tile walks replay their record; the wide walk keeps none
@@ -1808,7 +1808,7 @@ static sj_status launch_join(sj_grid_s *g, const JoinArgs &a, int pass, int prec
         return launch_join_mfma(ar, pass, g->ctx->cu_count, s, true);
     }
     JoinKernel kfn;
-    if (a.spanG > 0) kfn = pick_span(g->k, pass, prec, replay, a.spanDense != 0);
+    if (a.spanG > 0) kfn = pick_span(a, pass, prec, replay);
     else if (a.posLB && g->k == g->d && g->k == 2) kfn = pick_dense2(pass, prec, replay);
     else kfn = replay ? pick_replay(g->k, prec) : pick_kernel(g->k, g->d, pass, prec);
     if (!kfn) {

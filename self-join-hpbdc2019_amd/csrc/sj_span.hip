@@ -3,14 +3,14 @@
 
 namespace sj {
 
-template <int K, int PASS, bool F32, bool DENSE>
+template <int K, int PASS, bool F32, int MODE>
 __global__ __launch_bounds__(JB) __attribute__((amdgpu_waves_per_eu(F32 && K == 4 ? 4 : 3))) void k_span(JoinArgs a) {
     __shared__ SpanLds lds[WPB];
     if (PASS == PASS_FILL && !fill_gate(a)) return;
     LaneStats st;
     TileRec R;
     tile_loop<PASS>(a, st, R, [&](uint32_t tile) __attribute__((always_inline)) {
-        process_span<K, PASS, F32, DENSE>(a, tile, lds[threadIdx.x >> 6], st, R);
+        process_span<K, PASS, F32, MODE>(a, tile, lds[threadIdx.x >> 6], st, R);
     });
 }
 
@@ -26,27 +26,32 @@ __global__ __launch_bounds__(JB) void k_span_rp(JoinArgs a) {
     });
 }
 
-template <int K, bool DENSE>
+template <int K, int MODE>
 static JoinKernel pick_k(int pass, int prec) {
-    if (pass == PASS_COUNT) return prec ? k_span<K, PASS_COUNT, true, DENSE> : k_span<K, PASS_COUNT, false, DENSE>;
-    return prec ? k_span<K, PASS_FILL, true, DENSE> : k_span<K, PASS_FILL, false, DENSE>;
+    if constexpr (MODE == SPAN_DIRECT)  // no filter, so no precision of one
+        return pass == PASS_COUNT ? k_span<K, PASS_COUNT, false, MODE> : k_span<K, PASS_FILL, false, MODE>;
+    else if (pass == PASS_COUNT)
+        return prec ? k_span<K, PASS_COUNT, true, MODE> : k_span<K, PASS_COUNT, false, MODE>;
+    else
+        return prec ? k_span<K, PASS_FILL, true, MODE> : k_span<K, PASS_FILL, false, MODE>;
 }
 
-template <bool DENSE>
+template <int MODE>
 static JoinKernel pick(int k, int pass, int prec) {
     switch (k) {
-    case 4: return pick_k<4, DENSE>(pass, prec);
-    case 5: return pick_k<5, DENSE>(pass, prec);
-    case 6: return pick_k<6, DENSE>(pass, prec);
-    case 7: return pick_k<7, DENSE>(pass, prec);
-    case 8: return pick_k<8, DENSE>(pass, prec);
+    case 4: return pick_k<4, MODE>(pass, prec);
+    case 5: return pick_k<5, MODE>(pass, prec);
+    case 6: return pick_k<6, MODE>(pass, prec);
+    case 7: return pick_k<7, MODE>(pass, prec);
+    case 8: return pick_k<8, MODE>(pass, prec);
     }
     return nullptr;
 }
 
-JoinKernel pick_span(int k, int pass, int prec, bool replay, bool dense) {
+JoinKernel pick_span(const JoinArgs &a, int pass, int prec, bool replay) {
     if (replay) return k_span_rp;
-    return dense ? pick<true>(k, pass, prec) : pick<false>(k, pass, prec);
+    if (a.spanDirect) return pick<SPAN_DIRECT>(a.k, pass, prec);
+    return a.spanDense ? pick<SPAN_BLOCKS>(a.k, pass, prec) : pick<SPAN_FILTER>(a.k, pass, prec);
 }
 
 }  // namespace sj

@@ -629,7 +629,7 @@ struct SpanBand {
 SpanBand span_band(double T, double R, int k, bool f32);
 using JoinKernel = void (*)(JoinArgs);
 // Kernel of the span walk (sj_span.hip): count, evaluating or replaying fill.
-JoinKernel pick_span(int k, int pass, int prec, bool replay, bool dense);
+JoinKernel pick_span(const JoinArgs &a, int pass, int prec, bool replay);
 // Chooses the span walk for joins with d = k >= 4 and sets its fields.
 sj_status span_setup(sj_grid_s *g, JoinArgs &a, int prec);
 

@@ -2524,8 +2524,11 @@ __global__ void k_row_lengths_orig(const uint64_t *off, const uint32_t *rowIds, 
 // 16 lanes per row: rows are a few tens of IDs, and what bounds the copy is
 // the chain of loads in front of each row, so more rows in flight help
 // (64 lanes -> 16: 24M IDs in rows of 46 112 -> 59 us, 0.9M in rows of 9
-// 20 -> 8 us).
-constexpr int CR_LANES = 16;
+// 20 -> 8 us).  Eight IDs per lane are loaded together: one at a time, a few
+// long rows took longer than with 64 lanes (1,000 rows of 1,000 read as CSR:
+// 33 us with 64 lanes, 51 with 16, 28 with 16 x 8; 1.28M rows of 128: 616,
+// 396, 317 us).
+constexpr int CR_LANES = 16, CR_U = 8;
 __global__ __launch_bounds__(JB) void k_copy_rows_orig(const uint64_t *off, const int32_t *ids,
                                                        const uint32_t *rowIds, uint64_t n,
                                                        const uint64_t *offO, int32_t *idsO) {
@@ -2533,7 +2536,14 @@ __global__ __launch_bounds__(JB) void k_copy_rows_orig(const uint64_t *off, cons
     if (r >= n) return;
     const uint64_t b = off[r], e = off[r + 1];
     const uint64_t d = offO[rowIds[r]];
-    for (uint64_t i = b + threadIdx.x % CR_LANES; i < e; i += CR_LANES) idsO[d + (i - b)] = ids[i];
+    for (uint64_t i = b + threadIdx.x % CR_LANES; i < e; i += CR_LANES * CR_U) {
+        int32_t v[CR_U];
+#pragma unroll
+        for (int u = 0; u < CR_U; u++) v[u] = i + CR_LANES * u < e ? ids[i + CR_LANES * u] : 0;
+#pragma unroll
+        for (int u = 0; u < CR_U; u++)
+            if (i + CR_LANES * u < e) idsO[d + (i + CR_LANES * u - b)] = v[u];
+    }
 }
 
 sj_status result_to_orig(sj_result_s *r) {

@@ -2111,7 +2111,11 @@ sj_status join(sj_grid_s *g, const sj_join_params *P, sj_result_s *r) {
     uint64_t dirCap = 0, maskCap = 0;
     if (recording) {
         dirCap = span ? 0 : std::max<uint64_t>(ctx->recDirCap, std::max<uint64_t>(1ull << 20, n));
-        maskCap = std::max<uint64_t>(ctx->recMaskCap, std::max<uint64_t>(1ull << 23, 16 * n));
+        // words at first: masks need about 16 per point; the span walk's hits
+        // one each, so up to 64 neighbours per point (32 with the full
+        // stencil) fit, within 2 GiB
+        const uint64_t first = span ? std::max<uint64_t>(16 * n, std::min<uint64_t>(32 * n, 1ull << 28)) : 16 * n;
+        maskCap = std::max<uint64_t>(ctx->recMaskCap, std::max<uint64_t>(1ull << 23, first));
         bool room = recMask.alloc(pool, maskCap) == SJ_OK && recCtr.alloc(pool, REC_NCTR) == SJ_OK;
         if (span)
             room = room && recStart.alloc(pool, tBound) == SJ_OK && recN.alloc(pool, tBound) == SJ_OK;

@@ -205,20 +205,18 @@ __device__ __forceinline__ void process_point(const JoinArgs &a, uint32_t s, Lan
 }
 
 // ------------------------------------------------------------ tile path
-template <int D, int PREC>
 struct TileCfg {
-    static constexpr int DD = D > 0 ? D : 1;
-    static constexpr int CH = 256;  // staged candidates per chunk
-    static constexpr int MW = CH / 64;                              // mask words per lane (<= 4)
+    static constexpr int CH = 256;      // staged candidates per chunk
+    static constexpr int MW = CH / 64;  // mask words per lane
 };
 
 // Staged rows are padded by 64: a lane reads the 64 rows after its piece
 // start, masking the rows beyond its span.
 template <int D, int PREC>
 struct TileLds {
-    using C = TileCfg<D, PREC>;
-    double x64[PREC == 1 ? 1 : C::CH + 64][C::DD];
-    float x32[PREC == 1 ? C::CH + 64 : 1][C::DD];
+    using C = TileCfg;
+    double x64[PREC == 1 ? 1 : C::CH + 64][D];
+    float x32[PREC == 1 ? C::CH + 64 : 1][D];
     int32_t id[C::CH];
     uint32_t cnt[C::CH];
     unsigned long long base[C::CH];
@@ -234,7 +232,7 @@ constexpr uint32_t OWN_STAGE = 384;
 // row, with sdst[i] = l * 64 + t.
 template <int D, int PREC>
 struct TileLdsIds {
-    using C = TileCfg<D, PREC>;
+    using C = TileCfg;
     int32_t id[C::CH];
     uint32_t cnt[C::CH];
     unsigned long long base[C::CH];
@@ -249,9 +247,9 @@ struct TileLdsIds {
 template <int K, int D, int PASS, int PREC, bool RP, class LDS, bool DN = false>
 __device__ __forceinline__ void process_tile(const JoinArgs &a, uint32_t tile, LDS &L, LaneStats &st,
                                              TileRec &R) {
-    using Cfg = TileCfg<D, PREC>;
+    using Cfg = TileCfg;
     constexpr int CH = Cfg::CH;
-    constexpr int DD = Cfg::DD;
+    constexpr int DD = D;
     static_assert(!RP || PASS == PASS_FILL, "only the fill replays a record");
     const unsigned lane = __lane_id();
     const uint32_t ts0 = a.tileStart[tile], ts1 = a.tileStart[tile + 1];
@@ -856,8 +854,7 @@ __global__ __launch_bounds__(JB) void k_join_rp(JoinArgs a) {
     join_body<K, D, PASS_FILL, PREC, true, TileLdsIds<D, PREC>, DN>(a, lds);
 }
 
-// k <= 2: five waves per SIMD (at most 96 VGPRs); measured faster at 2-D,
-// slower at 6-D
+// k <= 2: five waves per SIMD (at most 96 VGPRs); measured faster at 2-D
 template <int K, int D, int PREC, bool DN = false>
 __global__ __launch_bounds__(JB) __attribute__((amdgpu_waves_per_eu(5))) void k_join_rp_o5(JoinArgs a) {
     __shared__ TileLdsIds<D, PREC> lds[WPB];
@@ -867,10 +864,9 @@ __global__ __launch_bounds__(JB) __attribute__((amdgpu_waves_per_eu(5))) void k_
 // ------------------------------------------------------------ many joins
 // One persistent launch over the tiles of many independent joins: work
 // item w is tile workTile[w] of instance workInst[w], whose arguments are
-// args[instance].  FP32 instances run the FP32 LDS tile walk when
-// d == k <= 8 and the matrix-core walk otherwise; FP64 ones the LDS tile
-// walk when d == k <= 8 and the wide walk otherwise.  Statistics go to the
-// instance's counters.
+// args[instance].  Instances with d == k run the LDS tile walk up to k = 3 and
+// the span walk from 4 to 8; the others the matrix-core walk in FP32 and the
+// wide walk in FP64.  Statistics go to the instance's counters.
 template <int A, int B>
 struct cmax {
     static constexpr int v = A > B ? A : B;
@@ -887,8 +883,8 @@ struct LdsMax<0> {
     static constexpr int v = cmax<(int)sizeof(WideLds), (int)sizeof(MfmaLds<64>)>::v;
 };
 constexpr int MANY_LDS = (cmax<LdsMax<SPAN_MINK - 1>::v, (int)sizeof(SpanLds)>::v + 15) / 16 * 16;
-// FP32 instances none of which uses the matrix cores: the FP32 LDS tile
-// walks only
+// FP32 instances none of which has d != k or d > 8: the FP32 LDS tile walks and
+// the span walk only
 template <int D>
 struct LdsMax32 {
     static constexpr int v =
@@ -1564,7 +1560,6 @@ JoinArgs base_args(sj_grid_s *g, int form, double T) {
     a.qEnd = (uint32_t)g->n;
     a.wBegin = 0;
     a.wEnd = (uint32_t)g->n;
-    a.nPts = (uint32_t)g->n;
     return a;
 }
 
@@ -1966,9 +1961,9 @@ static sj_status sample_count_list(sj_grid_s *g, const uint32_t *list, uint64_t 
 sj_status sort_rows_device(sj_context ctx, const uint64_t *offsets, int32_t *ids, uint64_t n, uint64_t base,
                            uint64_t idsCap = 0);
 
-// Decision constants of the precision form.  The FP32 LDS tile walk
-// (d == k <= 8) centres each tile in FP64 and sets its band per tile: it
-// needs nothing here.  The others use an FP32 copy relative to the grid
+// Decision constants of the precision form.  The FP32 LDS tile walk (d == k <= 3)
+// centres each tile in FP64 and sets its band per tile, and the span walk
+// (4 to 8) has its own constants: neither needs anything here.  The others use an FP32 copy relative to the grid
 // origin and its largest coordinate (one host sync): the matrix cores
 // (d > 8 or d != k, d <= 64) stage from that copy when the coordinates lie
 // within 1024 eps of the origin and centre each tile in FP64 otherwise; the

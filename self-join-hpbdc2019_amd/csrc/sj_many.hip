@@ -339,7 +339,7 @@ sj_status plan(sj_many_s *m, const sj_instance *in, int count) {
     m->W = (uint32_t)W;
     m->mfma = P.precision == SJ_PREC_FP32_RECHECK ? 1 : 0;
     if (m->mfma) {
-        // no instance on the matrix cores: the FP32 LDS tile walks only
+        // no instance with d != k or d > 8: the FP32 tile and span walks only
         bool anyMfma = false;
         for (int i = 0; i < count; i++) anyMfma = anyMfma || m->args[i].mDP > 0;
         if (!anyMfma) m->mfma = 2;

@@ -10,8 +10,8 @@
 // first cell's linear ID minus M = sum of the multipliers of dims < g to the
 // last cell's plus M, moved by the group's offset and cut to the group.
 //
-// All 64 x 64 pairs of the tile and a 64-candidate piece of the span go
-// through a filter on the matrix cores (v_mfma_*_16x16x4, FP64, or FP32 for
+// All pairs of the tile and 16 candidates of the span at a time go through a
+// filter on the matrix cores (v_mfma_*_16x16x4, FP64, or FP32 for
 // the FP32+recheck form): with y = x - (the tile's first point), rounded
 // once, |q|^2 + |c|^2 - 2 q.c <= T, where the products are the matrix
 // instructions, |q|^2 is their accumulator input and |c|^2 sits in the
@@ -140,8 +140,7 @@ __device__ __forceinline__ uint32_t pk_diff(uint32_t b, uint32_t a) { return ((b
 // Any field equal to 2: the cells are not adjacent.
 __device__ __forceinline__ bool pk_far(uint32_t z) { return (z & ~(z << 1) & 0x22222222u) != 0u; }
 
-// The span of a tile inside its own group: [lo, hi) linear IDs, the group's
-// base and the sum of multipliers.
+// The span of a tile inside its own group: linear IDs [lo, hi).
 struct TileSpan {
     uint64_t lo, hi;
 };

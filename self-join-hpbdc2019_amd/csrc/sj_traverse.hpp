@@ -60,7 +60,7 @@ struct JoinArgs {
     uint64_t outBase;
     unsigned long long *mirCur;
     int32_t *ids;
-    // hit record (LDS tile walk): the count pass stores, per executed
+    // hit record (all walks but the span walk's, below): the count pass stores, per executed
     // 64-candidate piece, a directory entry {lanes with hits, first mask
     // word} and the hit masks of those lanes back to back; the fill replays
     // them instead of evaluating distances again.  recDir null: no record.
@@ -72,7 +72,6 @@ struct JoinArgs {
     // span walk (spanG > 0): tiles are runs of points of one group of cells
     // with the same coordinates in dims spanG..k-1 (spanG = 0: one cell row)
     int spanG;
-    uint32_t nPts;             // points in the sorted arrays
     int spanDirect;            // no filter: the predicate for every candidate
     int spanDense;             // kernels that decide blocks with many hits whole
     double spanScale, spanT1;  // filter: norms scaled by 1 - alpha, threshold

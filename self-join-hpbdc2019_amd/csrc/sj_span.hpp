@@ -404,6 +404,16 @@ __device__ __forceinline__ bool span_plain32(const JoinArgs &a, uint32_t ts0, co
     return s32 <= (float)a.T;
 }
 
+// Whether the plain FP32 decision of a pair at d2 can differ from the exact one:
+// its sum errs by at most (2.03 K + 8.02) u s (span_band), s = |q|^2 + |c|^2 <=
+// 3 |q|^2 + 2 d2, and fl32(T) by u T; 1.1 covers nq, |q|^2 scaled, and the rest.
+// Few pairs are that near eps: deciding all of them took 5% of the 6-D count.
+template <int K>
+__device__ __forceinline__ bool span_plain_unsure(const JoinArgs &a, double d2, float nq) {
+    constexpr double u = 1.1 * 0x1p-24;
+    return fabs(d2 - a.T) <= u * ((2.03 * K + 8.02) * (3.0 * (double)nq + 2.0 * d2) + a.T);
+}
+
 // Decides the nh <= 64 gathered pairs from buffer position head, one per
 // lane, and counts and records them, or writes them to their rows.
 template <int K, int PASS, bool F32, int MODE>
@@ -428,10 +438,12 @@ __device__ __forceinline__ void span_flush(const JoinArgs &a, SpanLds &L, uint32
         for (int j = 0; j < K; j++) ok = ok && cc[j] - cq[j] + 1u <= 2u;
     }
     if (ok) {
-        ok = d2_fp64<K>(xq, xc, K) <= a.T;
+        const double d2 = d2_fp64<K>(xq, xc, K);
+        ok = d2 <= a.T;
         if (F32 && PASS == PASS_COUNT && !span_direct<MODE>(a)) {
             st.band++;
-            st.mis += ok != span_plain32<K>(a, ts0, xq, xc) ? 1u : 0u;
+            if (MODE == SPAN_ANY || span_plain_unsure<K>(a, d2, reinterpret_cast<const float *>(L.nq)[q]))
+                st.mis += ok != span_plain32<K>(a, ts0, xq, xc) ? 1u : 0u;
         }
     }
     const uint64_t okm = __ballot(ok);

@@ -105,6 +105,32 @@ def test_filter_passes_what_plain_fp32_accepts(d, eps, mult):
         assert ok[accepted].all()
 
 
+@pytest.mark.parametrize("d,eps,mult", CASES)
+def test_plain_fp32_errs_only_near_eps(d, eps, mult):
+    """the count of wrong plain FP32 decisions looks only at pairs whose d2 is
+    within u ((2.03 d + 8.02) (3 nq + 2 d2) + T) of T, u = 1.1 * 2^-24, nq the
+    query's scaled norm"""
+    rng = np.random.default_rng(5000 + d)
+    T = O.eps_threshold(eps)
+    centre = rng.uniform(-mult * eps, mult * eps, size=d)
+    dirs = rng.normal(size=(200_000, d))
+    dirs /= np.linalg.norm(dirs, axis=1, keepdims=True)
+    p = rng.uniform(-mult * eps, mult * eps, size=dirs.shape)
+    q = p + dirs * (eps * (1.0 + rng.uniform(-4e-6, 4e-6, size=(len(dirs), 1)) * mult))
+    A, B = (p - centre).astype(np.float32), (q - centre).astype(np.float32)
+    f = B - A
+    s32 = f[:, 0] * f[:, 0]
+    for j in range(1, d):
+        s32 = fma32(f[:, j], f[:, j], s32)
+    d2 = O.dist2_batch(p, q)
+    wrong = (s32 <= np.float32(T)) != (d2 <= T)
+    assert wrong.any()
+    _, scale, _ = sjamd.span_band(T, 4.0 * mult * eps + 2.0 * eps, d, sjamd.FP32_RECHECK)
+    nq = (_norm(A) * np.float32(scale)).astype(np.float64)
+    near = np.abs(d2 - T) <= 1.1 * 2.0 ** -24 * ((2.03 * d + 8.02) * (3.0 * nq + 2.0 * d2) + T)
+    assert near[wrong].all()
+
+
 @pytest.mark.parametrize("prec", [sjamd.FP64, sjamd.FP32_RECHECK])
 def test_filter_range(prec):
     """outside its range every pair goes to the predicate; inside it the

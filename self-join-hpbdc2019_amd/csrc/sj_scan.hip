@@ -170,8 +170,8 @@ sj_status scan_two_pass(Pool *pool, hipStream_t s, In in, uint64_t n, Tacc *out)
     }
     DBuf<Tacc> sums;
     SJ_TRY(sums.alloc(pool, nb));
-    // a single tile has no tiles before it: one launch (1,000 points: four
-    // scans, 246 -> 211 us a join)
+    // a single tile has no tiles before it: one launch instead of two (four of
+    // about 28 in a join of 1,000 points, within the noise of its 224 to 232 us)
     if (nb > 1) {
         hipLaunchKernelGGL((k_tile_sums<In, Tacc>), dim3((unsigned)nb), dim3(SB), 0, s, in, n, sums.p);
         SJ_LAUNCH_CHECK();

@@ -42,13 +42,13 @@
 // REC_BLK words, whose last word links to the next block; recN counts them.
 // The replaying fill reads up to 256 words at a time and looks nothing up.
 // Bound: latency.  2M points uniform in 6-D, FP32+recheck: 9.4e9 pairs in
-// 3.6 ms, of which the matrix instructions are busy 1.05 ms and the vector
-// instructions 1.2 ms; 157 registers allow three waves per SIMD, and half of
-// their time they wait (candidates' loads, compare to branch, the gathered
-// pairs' loads and atomics).  Measured against the row walk with LDS-staged
-// windows it replaced (count, replayed fill): that case 6.94, 4.11 -> 3.60,
-// 0.73 ms; 100,000 points in 8-D, FP64 6.23, 1.73 -> 1.22, 0.04 ms; 12 joins in
-// 2 to 8 dims in one graph 39.0, 33.1 ms -> 2.9 ms for both.  Tried and left: the candidates
+// 3.8 ms, of which the matrix instructions are busy 1.05 ms and the vector
+// instructions 1.2 ms (profiles/counters_span_mfma.md); 147 registers allow
+// three waves per SIMD, and 46% of their cycles they wait (candidates' loads,
+// the gathered pairs' loads and atomics).  Measured against the row walk with
+// LDS-staged windows it replaced (count, replayed fill): that case 6.94, 4.11
+// -> 3.84, 0.55 ms; 100,000 points in 8-D, FP64 6.23, 1.73 -> 1.25, 0.02 ms; 12
+// joins in 2 to 8 dims in one graph 39.0, 33.1 ms -> 2.8 ms for both.  Tried and left: the candidates
 // as scalar operands of vector FMAs (8.3 ms in 6-D, waiting for the scalar
 // cache), hit masks per lane and 64-candidate piece instead of gathered pairs
 // (5.9 ms, fill 1.2 ms), loads four steps ahead (4.1 ms: more registers).

@@ -43,7 +43,7 @@
 // The replaying fill reads up to 256 words at a time and looks nothing up.
 // Bound: latency.  2M points uniform in 6-D, FP32+recheck: 9.4e9 pairs in
 // 3.8 ms, of which the matrix instructions are busy 1.05 ms and the vector
-// instructions 1.2 ms (profiles/counters_span_mfma.md); 147 registers allow
+// instructions 1.2 ms; 147 registers allow
 // three waves per SIMD, and 46% of their cycles they wait (candidates' loads,
 // the gathered pairs' loads and atomics).  Measured against the row walk with
 // LDS-staged windows it replaced (count, replayed fill): that case 6.94, 4.11
